@@ -233,10 +233,14 @@ struct mspms_ctx {
     const double* cur_rep_delt = nullptr;  // integrator kernels' per-replica
                                            // steps while an HMC move is enqueued
 
-    // Nose-Hoover NVT (mspms_nvt_set): states, the last solve's sum m v^2,
-    // the Newton iterate (3, N)
+    // Nose-Hoover NVT (mspms_nvt_set): states, the kernels' work lists, their
+    // workgroup sums and the thermostats between the kernels of a step
     DevBuf<mspms_nvt_state> d_nvt;
-    DevBuf<double> d_nvt_carry, d_nvt_vn;
+    DevBuf<int4> d_nvt_work_m, d_nvt_work_a;
+    DevBuf<int2> d_nvt_blk_m, d_nvt_blk_a;
+    DevBuf<double4> d_nvt_part;
+    DevBuf<NvtScal> d_nvt_scal;
+    NvtPlan nvt_plan{};
     DevBuf<int> d_active;                // replicas the NVT kernels advance
     bool nvt_ready = false;
     // NPT (mspms_npt_set)
@@ -623,8 +627,12 @@ extern "C" int mspms_destroy(mspms_ctx* c) {
     c->d_hmc_delt.release();
     c->d_nvt.release();
     c->d_npt.release();
-    c->d_nvt_carry.release();
-    c->d_nvt_vn.release();
+    c->d_nvt_work_m.release();
+    c->d_nvt_work_a.release();
+    c->d_nvt_blk_m.release();
+    c->d_nvt_blk_a.release();
+    c->d_nvt_part.release();
+    c->d_nvt_scal.release();
     c->d_active.release();
     if (c->h_status) (void)hipHostFree(c->h_status);
     if (c->side) (void)hipStreamSynchronize(c->side);
@@ -2127,24 +2135,29 @@ int enqueue_nvt(mspms_ctx* c, double* pos, double* vel, double* fl, double* fs, 
     const double deltby2 = delt / 2.0, delts = delt / nstep_inner, deltsby2 = delts / 2.0;
     const double delt_sqby2 = delt * delt / 2.0, delts_sqby2 = delts * delts / 2.0;
     LaunchCtx L = launch_ctx(c, s);
+    NvtArgs P{};
+    P.t = NvtTimes{delt, deltby2, delt_sqby2, delts, deltsby2, delts_sqby2};
+    P.n = n;
+    P.mols = c->d_mols.p;
+    P.terms = c->d_terms.p;
+    P.rmass = c->d_rmass.p;
+    P.st = c->d_nvt.p;
+    P.x = pos;
+    P.v = vel;
+    P.fl = fl;
+    P.fs = fs;
+    P.epart = c->d_ep_short.p;
+    P.active = c->d_active.p;
+    P.status = c->d_status.p;
     {
         ProfScope p(c, s, PROF_BONDED);
-        for (int ll = 0; ll < nstep_inner; ll++) {
-            launch_nvt_drift(L, c->d_nvt.p, ll == 0, pos, pos + n, pos + 2 * n, vel, vel + n,
-                             vel + 2 * n, fl, fs, deltby2, delts, deltsby2, delts_sqby2,
-                             c->d_active.p);
-            launch_bonded(L, c->d_species.p, c->d_terms.p, pos, pos + n, pos + 2 * n, fs, fs + n,
-                          fs + 2 * n, c->d_ep_short.p);
-            launch_nvt_solve(L, c->d_nvt.p, false, c->d_nvt_carry.p, vel, vel + n, vel + 2 * n,
-                             fs, c->d_nvt_vn.p, delts, deltsby2, delts_sqby2, nullptr,
-                             c->d_active.p);
-        }
+        for (int ll = 0; ll < nstep_inner; ll++)
+            launch_nvt_substep(L, c->nvt_plan, c->d_species.p, P, ll, ll == nstep_inner - 1);
     }
     int rc = enqueue_long(c, pos, pos + n, pos + 2 * n, fl, fl + n, fl + 2 * n, lterms, s,
                           nullptr, false);
     if (rc) return rc;
-    launch_nvt_solve(L, c->d_nvt.p, true, c->d_nvt_carry.p, vel, vel + n, vel + 2 * n, fl,
-                     c->d_nvt_vn.p, delt, deltby2, delt_sqby2, ukin, c->d_active.p);
+    launch_nvt_outer(L, c->nvt_plan, P, nstep_inner, ukin);
     {
         ProfScope p(c, s, PROF_FINAL);
         launch_finalize(c, L, lterms, sterms, nullptr);
@@ -2162,11 +2175,39 @@ extern "C" int mspms_nvt_set(mspms_ctx* c, const mspms_nvt_state* st) {
         if (!(st[r].qq > 0.0) || !(st[r].qqs > 0.0) || !(st[r].treq > 0.0) || st[r].nfree < 1)
             return fail(MSPMS_EINVAL, "replica %d: qq, qqs, treq and nfree must be positive", r);
     HIPC(hipSetDevice(c->device));
+    // the workgroups of the substep kernel (by molecules, where they fit it)
+    // and of the atom passes; every replica has at least one
+    std::vector<int4> work[2];
+    std::vector<int2> blk[2];
+    int most_atoms = 0;
+    for (const SpeciesHost& q : c->sp) most_atoms = std::max(most_atoms, q.natom);
+    const int per[2] = {nvt_mols_per_block(most_atoms, c->max_mol_terms), nvt_atoms_per_block()};
+    for (int k = 0; k < 2; k++) {
+        if (per[k] == 0) continue;
+        for (const RepDev& R : c->reps) {
+            const int first = k == 0 ? R.mol0 : R.atom0, cnt = k == 0 ? R.nmol : R.natom;
+            const int b0 = (int)work[k].size(), nb = std::max(1, (cnt + per[k] - 1) / per[k]);
+            for (int b = 0; b < nb; b++)
+                work[k].push_back(make_int4((int)(&R - c->reps.data()), first + b * per[k],
+                                            std::max(0, std::min(per[k], cnt - b * per[k])),
+                                            b == 0));
+            blk[k].push_back(make_int2(b0, nb));
+        }
+    }
+    const size_t npart = std::max(work[0].size(), work[1].size());
     int rc;
-    if ((rc = c->d_nvt.ensure(c->nrep)) || (rc = c->d_nvt_carry.ensure(c->nrep)) ||
-        (rc = c->d_nvt_vn.ensure((size_t)3 * c->natom)) ||
+    drop_graph(c);  // buffers may move
+    if ((rc = c->d_nvt.ensure(c->nrep)) || (rc = c->d_nvt_work_m.upload(work[0], c->stream)) ||
+        (rc = c->d_nvt_work_a.upload(work[1], c->stream)) ||
+        (rc = c->d_nvt_blk_m.upload(blk[0], c->stream)) ||
+        (rc = c->d_nvt_blk_a.upload(blk[1], c->stream)) ||
+        (rc = c->d_nvt_part.ensure(2 * npart)) ||
+        (rc = c->d_nvt_scal.ensure((size_t)2 * c->nrep)) ||
         (rc = c->d_active.upload(std::vector<int>(c->nrep, 1), c->stream)))
         return rc;
+    c->nvt_plan = NvtPlan{c->d_nvt_work_m.p, c->d_nvt_work_a.p, c->d_nvt_blk_m.p,
+                          c->d_nvt_blk_a.p,  (int)work[0].size(), (int)work[1].size(),
+                          c->d_nvt_part.p,   c->d_nvt_scal.p,     npart};
     HIPC(hipMemcpyAsync(c->d_nvt.p, st, sizeof(mspms_nvt_state) * c->nrep,
                         hipMemcpyHostToDevice, c->stream));
     HIPC(hipStreamSynchronize(c->stream));

@@ -302,16 +302,56 @@ void launch_npt_inner(const LaunchCtx& c, RepDev* reps, NptDev* st, bool first, 
                       double* vel, const double* fs, double delts, double deltsby2);
 void launch_kvec(const LaunchCtx& c, const RecipBufs& rb, int nrow);
 
-// Nose-Hoover NVT (k_nvt.hip), one workgroup per replica
+// Nose-Hoover NVT (k_nvt.hip)
 struct mspms_nvt_state;
-void launch_nvt_drift(const LaunchCtx& c, mspms_nvt_state* st, bool first, double* x, double* y,
-                      double* z, double* vx, double* vy, double* vz, const double* fl,
-                      const double* fs, double deltby2, double delts, double deltsby2,
-                      double delts_sqby2, const int* active);
-void launch_nvt_solve(const LaunchCtx& c, mspms_nvt_state* st, bool outer, double* carry,
-                      double* vx, double* vy, double* vz, const double* f, double* vn,
-                      double dt, double dtby2, double dt_sqby2, double* ukin,
-                      const int* active);
+// time steps of the outer step and the substep, as init_nvt derives them
+struct NvtTimes {
+    double delt, deltby2, delt_sqby2, delts, deltsby2, delts_sqby2;
+};
+// the thermostats between the kernels of a step; s2: sum m v^2
+struct NvtScal {
+    double ss, ps, sss, pss, s2;
+};
+// Work of the NVT kernels: (replica, first molecule or atom, count, 1 for
+// the replica's first workgroup) per workgroup, and per replica its
+// workgroups (first, count).  nwork_m is 0 where the molecules are too large
+// for the molecule-wise substep.  part, scal: two records each, alternating
+// from kernel to kernel.
+struct NvtPlan {
+    const int4 *work_m, *work_a;
+    const int2 *blk_m, *blk_a;
+    int nwork_m, nwork_a;
+    double4* part;   // [2][npart]
+    NvtScal* scal;   // [2][nrep]
+    size_t npart;
+};
+struct NvtArgs {
+    NvtTimes t;
+    size_t n;                  // atoms
+    const MolDev* mols;
+    const TermDev* terms;
+    const double* rmass;
+    mspms_nvt_state* st;
+    double *x, *v;             // (3, n)
+    const double* fl;
+    double* fs;
+    double* epart;
+    const int* active;         // replicas the kernels advance
+    Status* status;
+    // filled in per launch
+    const int4* work;
+    const int2* blk_in;
+    const double4* part_in;
+    double4* part_out;
+    const NvtScal* scal_in;
+    NvtScal* scal_out;
+};
+int nvt_mols_per_block(int max_mol_atoms, int max_mol_terms);
+int nvt_atoms_per_block();
+void launch_nvt_substep(const LaunchCtx& c, const NvtPlan& N, const SpeciesDev* species, NvtArgs P,
+                        int ll, int last);
+void launch_nvt_outer(const LaunchCtx& c, const NvtPlan& N, NvtArgs P, int nstep_inner,
+                      double* ukin);
 
 // [type][128][ncube] (the file's order) -> [type][cube][128]
 void launch_cube_major(hipStream_t s, const double* src, double* dst, int ntype, int ncube);
