@@ -160,11 +160,12 @@ struct mspms_ctx {
 
     // reciprocal
     RecipBufs rb{};
-    DevBuf<KRow> d_rows, d_rows_s;
-    DevBuf<double> d_kvec, d_uk;
-    DevBuf<int> d_k_rep, d_rep_chunk0;
+    DevBuf<KRow> d_rows;
+    DevBuf<KTileRow> d_trows;
+    DevBuf<double> d_kvec, d_uk, d_s_part, d_wmat;
+    DevBuf<int> d_tile_rep, d_rep_chunk0;
     DevBuf<int4> d_work_s, d_work_f;
-    DevBuf<double2> d_s_part, d_ak;
+    DevBuf<double2> d_w0;
 
     // partial sums and outputs
     DevBuf<double> d_ep_pair, d_ep_intra, d_ep_short, d_ep_sf, d_uvac, d_ep_coul;
@@ -585,15 +586,16 @@ extern "C" int mspms_destroy(mspms_ctx* c) {
     c->d_eatom.release();
     c->d_fslot.release();
     c->d_rows.release();
-    c->d_rows_s.release();
+    c->d_trows.release();
     c->d_kvec.release();
     c->d_uk.release();
-    c->d_k_rep.release();
+    c->d_tile_rep.release();
     c->d_rep_chunk0.release();
     c->d_work_s.release();
     c->d_work_f.release();
     c->d_s_part.release();
-    c->d_ak.release();
+    c->d_wmat.release();
+    c->d_w0.release();
     c->d_ep_pair.release();
     c->d_ep_intra.release();
     c->d_ep_short.release();
@@ -776,11 +778,12 @@ int build(mspms_ctx* c) {
             return fail(MSPMS_EINVAL, "simple Coulomb supports molecules of at most 16 sites");
     }
     c->any_sf = false;
-    std::vector<KRow> rows, rows_s;
+    std::vector<KRow> rows;
+    std::vector<KTileRow> trows;
     std::vector<double> kvec;
-    std::vector<int> k_rep, rep_chunk0(1, 0);
+    std::vector<int> tile_rep, rep_chunk0(1, 0);
     std::vector<int4> work_s, work_f;
-    int ntab_max = 1, nkz_max = 1, nk_stride = 1, nkrow_max = 1;
+    int kmax_all[3] = {0, 0, 0}, ntile_max = 1;
     size_t max_rep_cl = 1;
     double max_est = 0.0;
     for (int r = 0; r < c->nrep; r++) {
@@ -916,7 +919,6 @@ int build(mspms_ctx* c) {
                                    rkz = P.twopi_lz * kz;
                             volatile double rksq = rkx * rkx + rky * rky + rkz * rkz;
                             kvec.push_back(2.0 * (std::exp(-P.bfactor_ewald * rksq) / rksq));
-                            k_rep.push_back(r);
                             row.kz_hi = kz;
                             n++;
                         }
@@ -935,54 +937,51 @@ int build(mspms_ctx* c) {
                 }
             R.nkrow = (int)rows.size() - R.krow0;
             R.nk = (int)kvec.size() - R.k0;
-            nk_stride = std::max(nk_stride, R.nk);
-            ntab_max = std::max(ntab_max, P.kmaxx + P.kmaxy + std::max(P.kmaxz, 1) + 3);
-            nkz_max = std::max(nkz_max, 2 * P.kmaxz + 1);
-            nkrow_max = std::max(nkrow_max, R.nkrow);
-            // S pass: rows sorted by length; one workgroup per SK_CHUNK-atom
-            // chunk (the kernel's tables hold up to 64).  Smaller chunks give
-            // more waves but take more of the GPU from the pair kernel that
-            // runs beside this pass: 64 measured fastest for the RESPA step
+            kmax_all[0] = std::max(kmax_all[0], P.kmaxx);
+            kmax_all[1] = std::max(kmax_all[1], P.kmaxy);
+            kmax_all[2] = std::max(kmax_all[2], P.kmaxz);
+            // the rows in tiles of 8, longest kz extent first
             std::vector<KRow> rs(rows.begin() + R.krow0, rows.end());
-            std::stable_sort(rs.begin(), rs.end(),
-                             [](const KRow& a, const KRow& b) { return a.nk > b.nk; });
-            rows_s.insert(rows_s.end(), rs.begin(), rs.end());
-            const int SK_CHUNK = 64;
-            int nchunk = (R.natom + SK_CHUNK - 1) / SK_CHUNK;
-            for (int ch = 0; ch < nchunk; ch++) {
-                int a0 = R.atom0 + SK_CHUNK * ch;
-                work_s.push_back(make_int4(r, rep_chunk0.back() + ch, a0,
-                                           std::min(SK_CHUNK, R.atom0 + R.natom - a0)));
+            std::stable_sort(rs.begin(), rs.end(), [](const KRow& a, const KRow& b) {
+                return a.kz_hi > b.kz_hi;
+            });
+            R.ktile0 = (int)(trows.size() / 8);
+            R.nktile = ((int)rs.size() + 7) / 8;
+            for (int i = 0; i < 8 * R.nktile; i++) {
+                KTileRow t{};
+                t.nz = t.k0 = -1;
+                if (i < (int)rs.size()) {
+                    t.kx = rs[i].kx;
+                    t.ky = rs[i].ky;
+                    t.kz_lo = rs[i].kz_lo;
+                    t.nz = rs[i].kz_hi;
+                    t.k0 = rs[i].k0;
+                }
+                trows.push_back(t);
             }
-            rep_chunk0.push_back(rep_chunk0.back() + nchunk);
-        } else {
-            rep_chunk0.push_back(rep_chunk0.back());
+            tile_rep.insert(tile_rep.end(), R.nktile, r);
+            ntile_max = std::max(ntile_max, R.nktile);
         }
         if (P.iSF_type != MSPMS_SF_NONE) c->any_sf = true;
     }
+    const int f_group = recip_f_group((long)atom_mol.size());
     if (c->any_recip) {
-        // force pass: (atom block of 64) x (row group), ~4096 waves in total
-        const long KF_WAVES = 4096;
+        // the structure factor's atom chunks and the force pass's atom groups
         long blocks = 0;
-        for (int r = 0; r < c->nrep; r++) blocks += (reps[r].natom + 63) / 64;
+        for (int r = 0; r < c->nrep; r++)
+            if (reps[r].nktile > 0) blocks += (reps[r].natom + 63) / 64;
+        const int chunk = recip_s_chunk(blocks);
         for (int r = 0; r < c->nrep; r++) {
             const RepDev& R = reps[r];
-            int nb = (R.natom + 63) / 64;
-            int groups = (int)std::max(
-                1L, std::min((long)R.nkrow, (KF_WAVES + blocks - 1) / std::max(blocks, 1L)));
-            // split rows into `groups` ranges of about equal k count
-            std::vector<int> cut(1, R.krow0);
-            double per = (double)R.nk / groups, acc = 0.0;
-            for (int i = R.krow0; i < R.krow0 + R.nkrow; i++) {
-                acc += rows[i].nk;
-                if (acc >= per * (double)cut.size() && (int)cut.size() < groups && i + 1 < R.krow0 + R.nkrow)
-                    cut.push_back(i + 1);
+            if (R.nktile > 0) {
+                for (int a = 0; a < R.natom; a += chunk)
+                    work_s.push_back(make_int4(r, (int)work_s.size(), R.atom0 + a,
+                                               std::min(chunk, R.natom - a)));
+                for (int a = 0; a < R.natom; a += f_group)
+                    work_f.push_back(
+                        make_int4(r, R.atom0 + a, std::min(f_group, R.natom - a), 0));
             }
-            cut.push_back(R.krow0 + R.nkrow);
-            for (int b = 0; b < nb; b++)
-                for (size_t g = 0; g + 1 < cut.size(); g++)
-                    if (cut[g + 1] > cut[g])
-                        work_f.push_back(make_int4(r, R.atom0 + 64 * b, cut[g], cut[g + 1]));
+            rep_chunk0.push_back((int)work_s.size());
         }
     }
     c->natom = (int)atom_mol.size();
@@ -1061,33 +1060,39 @@ int build(mspms_ctx* c) {
     RecipBufs& R = c->rb;
     memset(&R, 0, sizeof R);
     if (c->any_recip) {
-        int nchunk = rep_chunk0.back();
-        if ((rc = c->d_rows.upload(rows, s)) || (rc = c->d_rows_s.upload(rows_s, s)) ||
-            (rc = c->d_kvec.upload(kvec, s)) || (rc = c->d_k_rep.upload(k_rep, s)) ||
+        const int nt = recip_kz_tiles(kmax_all[2]);
+        const size_t stride = (size_t)ntile_max * (256 * nt + 16), ntile = tile_rep.size();
+        if ((rc = c->d_rows.upload(rows, s)) || (rc = c->d_trows.upload(trows, s)) ||
+            (rc = c->d_kvec.upload(kvec, s)) || (rc = c->d_tile_rep.upload(tile_rep, s)) ||
             (rc = c->d_work_s.upload(work_s, s)) || (rc = c->d_work_f.upload(work_f, s)) ||
             (rc = c->d_rep_chunk0.upload(rep_chunk0, s)) ||
-            (rc = c->d_s_part.ensure((size_t)nchunk * nk_stride)) ||
-            (rc = c->d_ak.ensure(kvec.size())) || (rc = c->d_uk.ensure(kvec.size())) ||
-            (rc = c->d_eatom.ensure(3 * (size_t)c->natom)))
+            (rc = c->d_s_part.ensure(work_s.size() * stride)) ||
+            (rc = c->d_wmat.ensure(2 * ntile * 4 * nt * 64)) || (rc = c->d_w0.ensure(8 * ntile)) ||
+            (rc = c->d_uk.ensure(kvec.size())) || (rc = c->d_eatom.ensure(3 * (size_t)c->natom)))
             return rc;
+        // the force product's matrix is zero where a row has no k
+        HIPC(hipMemsetAsync(c->d_wmat.p, 0, 2 * ntile * 4 * nt * 64 * sizeof(double), s));
         R.rows = c->d_rows.p;
         R.nrow = (int)rows.size();
-        R.rows_s = c->d_rows_s.p;
+        R.trows = c->d_trows.p;
+        R.tile_rep = c->d_tile_rep.p;
+        R.ntile = (int)ntile;
+        R.ntile_max = ntile_max;
+        R.nt = nt;
+        R.kx_max = kmax_all[0];
+        R.ky_max = kmax_all[1];
         R.kvec = c->d_kvec.p;
-        R.k_rep = c->d_k_rep.p;
         R.work_s = c->d_work_s.p;
         R.nwork_s = (int)work_s.size();
         R.work_f = c->d_work_f.p;
         R.nwork_f = (int)work_f.size();
+        R.f_group = f_group;
         R.rep_chunk0 = c->d_rep_chunk0.p;
         R.s_part = c->d_s_part.p;
-        R.nk_stride = nk_stride;
-        R.ak = c->d_ak.p;
+        R.s_stride = stride;
+        R.wmat = c->d_wmat.p;
+        R.w0 = c->d_w0.p;
         R.uk = c->d_uk.p;
-        R.nk_total = (int)kvec.size();
-        R.ntab_max = ntab_max;
-        R.nkz_max = nkz_max;
-        R.nkrow_max = nkrow_max;
         R.eatom = c->d_eatom.p;
     }
     // ---- solid-fluid tables (replica 0's model, shared) ----
@@ -1463,7 +1468,7 @@ int enqueue_long(mspms_ctx* c, const double* x, const double* y, const double* z
         }
         if (recip_side) {
             ProfScope p(c, c->side, PROF_RECIP_F);
-            launch_recip_f(Ls, c->rb, x, y, z, frec, frec + n, frec + 2 * n, nullptr);
+            launch_recip_f(Ls, c->rb, frec, frec + n, frec + 2 * n, nullptr);
         }
         HIPC(hipEventRecord(c->ev_join, c->side));
     }
@@ -1511,7 +1516,7 @@ int enqueue_long(mspms_ctx* c, const double* x, const double* y, const double* z
     if (c->any_recip) {
         if (!recip_side) {
             ProfScope p(c, s, PROF_RECIP_F);
-            launch_recip_f(L, c->rb, x, y, z, fx, fy, fz, gq);
+            launch_recip_f(L, c->rb, fx, fy, fz, gq);
         }
         if (c->any_vacuum)
             launch_vacuum(L, c->d_species.p, x, y, z, fx, fy, fz, c->d_uvac.p, gq);

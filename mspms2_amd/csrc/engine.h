@@ -64,6 +64,7 @@ struct RepDev {
     double h[3], inv_h[3];
     // Ewald reciprocal work tables (per replica ranges)
     int krow0, nkrow, k0, nk;
+    int ktile0, nktile;       // tiles of 8 sorted rows (KTileRow)
     int kmax[3], ksqmax;
     double twopi_over_3v;     // vacuum boundary term, src/initvars.c:441
     int ewald_bc, pad3;
@@ -76,6 +77,14 @@ struct KRow {
     int rep;
     int nk;                   // number of k in the row
     int pad;
+};
+
+// A row in the order of the reciprocal kernels' row tiles: longest kz extent
+// first within a replica, padded to a multiple of 8 by rows without k (k0 -1)
+struct KTileRow {
+    int kx, ky, kz_lo;
+    int nz;                   // largest kz (0: kz = 0 alone; -1 in padding rows)
+    int k0, pad[3];
 };
 
 // the three groups of scratch used by one frclong evaluation
@@ -211,21 +220,25 @@ struct LaunchCtx {
 
 struct RecipBufs {
     KRow* rows;          // reference order, per replica ranges
-    KRow* rows_s;        // same rows sorted by length (S pass)
+    int nrow;            // rows of all replicas
+    KTileRow* trows;     // [8 ntile]
+    int* tile_rep;       // [ntile]
+    int ntile, ntile_max;  // row tiles of all replicas; most of one replica
+    int nt;              // kz tiles of 8
+    int kx_max, ky_max;  // largest kmaxx, kmaxy of the replicas
     double* kvec;        // [nk_total] exp(-B k^2)/k^2 (host libm)
-    int* k_rep;          // [nk_total]
     int4* work_s;        // (rep, chunk, first atom, atoms)
     int nwork_s;
-    int4* work_f;        // (rep, first atom, first row, end row)
-    int nwork_f;
+    int4* work_f;        // (rep, first atom, atoms, -)
+    int nwork_f, f_group;
     int* rep_chunk0;     // [nrep+1]
-    double2* s_part;     // [nchunk][nk_stride]
-    int nk_stride;
-    double2* ak;         // [nk_total] force coefficients
+    double* s_part;      // [nchunk][s_stride]: per row tile, kz tile and result
+                         //   register 64 lanes; then 16 sums of n = 0 per tile
+    size_t s_stride;
+    double* wmat;        // [2 ntile][4 nt][64] the force product's left matrix
+                         //   (tiles of 4 rows), zero where a row has no k
+    double2* w0;         // [2 ntile][4] its n = 0 column
     double* uk;          // [nk_total] kvec |S|^2
-    int nk_total, ntab_max, nkz_max;
-    int nrow;            // rows of all replicas
-    int nkrow_max;       // most rows of one replica
     double2* eatom;      // [3][natom] exp(i 2 pi x_d / L_d) per atom and axis,
                          //   written by k_sk, read by k_kforce
 };
@@ -426,11 +439,12 @@ void launch_bonded(const LaunchCtx& c, const SpeciesDev* species,
                    const TermDev* terms, const double* x, const double* y,
                    const double* z, double* fx, double* fy, double* fz,
                    double* epart);
-int recip_nkz_supported(int kmaxz);
+int recip_kz_tiles(int kmaxz);
+int recip_s_chunk(long blocks64);
+int recip_f_group(long natom);
 void launch_recip_s(const LaunchCtx& c, const RecipBufs& rb, const double* x,
                     const double* y, const double* z);
-void launch_recip_f(const LaunchCtx& c, const RecipBufs& rb, const double* x,
-                    const double* y, const double* z, double* fx, double* fy,
+void launch_recip_f(const LaunchCtx& c, const RecipBufs& rb, double* fx, double* fy,
                     double* fz, double* gq = nullptr);
 // per (replica, site): sum of the per-atom derivatives over the replica's
 // atoms of that site, plus the self-energy term -2 q C coef (Ewald / Wolf)
