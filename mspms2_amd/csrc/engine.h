@@ -104,7 +104,7 @@ struct ClusterBufs {
     int* ncl_total;      // [1]
     int* slot_orig;      // [8*maxcl]
     int2* slot_info;     // [8*maxcl] (mol, site)
-    double4* slot_x64;   // [8*maxcl] FP64 unwrapped (x,y,z,-), current call
+    double4* slot_x64;   // [8*maxcl] FP64 unwrapped (x,y,z), current call, and charge
     double4* slot_w64;   // [8*maxcl] FP64 wrapped at the last build (x,y,z,charge)
     double4* atom_x0;    // [natom] unwrapped position at the last build
     int* lstate;         // [LS_N] list state: LS_VALID, LS_NEED (rebuild

@@ -102,7 +102,10 @@ __global__ void __launch_bounds__(64) k_list_check(
     const float BIG = 3.0e38f;
     float lo[3] = {BIG, BIG, BIG}, hi[3] = {-BIG, -BIG, -BIG};
     if (live_cl) {
-        slot_x64[t] = make_double4(xo, yo, zo, 0.0);
+        // (the charge in .w stays as the build left it)
+        double* px = reinterpret_cast<double*>(&slot_x64[t]);
+        *reinterpret_cast<double2*>(px) = make_double2(xo, yo);
+        px[2] = zo;
         const float4 off = make_float4((float)((w.x - C.x) + (xo - p0o.x)),
                                        (float)((w.y - C.y) + (yo - p0o.y)),
                                        (float)((w.z - C.z) + (zo - p0o.z)), (float)w.w);
@@ -392,7 +395,7 @@ __device__ inline void place_atom(int i, int col, int colstart, const double* __
     if (!(isfinite(xi) && isfinite(yi) && isfinite(zi))) xi = yi = zi = 0.0;
     slot_orig[slot] = i;
     slot_info[slot] = make_int2(atom_mol[i], atom_site[i]);
-    slot_x64[slot] = make_double4(x[i], y[i], z[i], 0.0);
+    slot_x64[slot] = make_double4(x[i], y[i], z[i], sites[atom_site[i]].charge);
     slot_w64[slot] = make_double4(wrap(xi, R.L[0], R.invL[0]), wrap(yi, R.L[1], R.invL[1]), wz,
                                   (double)sites[atom_site[i]].charge_f);
     atom_x0[i] = make_double4(x[i], y[i], z[i], 0.0);

@@ -19,8 +19,9 @@
 // Precision modes:
 //   FP64   separation from the unwrapped FP64 positions with the reference's
 //          minimum image (d - L*rint(d/L), true division, no contraction),
-//          reference-order FP64 terms: the (i<j, r<rc) pair sets are those of
-//          src/frclong.c:114-125 bit for bit.
+//          FP64 terms (LJ in the reference's order, Ewald and Wolf with the
+//          branch-free erfc of physics.h): the (i<j, r<rc) pair sets are
+//          those of src/frclong.c:114-125 bit for bit.
 //   MIXED  separation = (FP32 offset_i - offset_j) + (cluster-centre delta
 //          and image shift, FP64 rounded once to FP32); FP32 terms with the
 //          polynomial erfc; FP64 accumulation of forces, energies, virial.
@@ -61,148 +62,271 @@ __device__ inline int xcd_block(int b, int nb) {
     return lb;
 }
 
-// Exact mode (FP64, the reference's operation order), WPC waves per
-// i-cluster combined through LDS in wave order; GRAD adds the per-atom
-// parameter derivatives.
-template <int ELEC, bool FP64, bool GRAD, int WPC>
-__global__ void __launch_bounds__(64 * WPC) k_pair(
+// Exact mode (FP64), WPC waves per i-cluster combined through LDS in wave
+// order; GRAD adds the per-atom parameter derivatives.
+//
+// The FP64 terms cost several hundred cycles per wave, and only about a
+// third of an entry's 8 x 8 lanes hold a pair in range.  So a wave works in
+// two phases: per entry an FP32 test from the cluster offsets (as
+// k_pair_mx's geometry) with a margin above its rounding, whose survivors
+// go to a queue in LDS; and, once some atom of the i-cluster has more than
+// 24 queued, one evaluation of up to eight per atom: lane (i, k) takes i's
+// k-th.  The evaluation forms the separation from the FP64 positions as the
+// reference does and decides by its own r^2 < rc^2, so the pair sets are
+// those of src/frclong.c:114-125 whatever the first test let through.  An
+// atom's lanes stay its own, so forces need no atomics and their order is
+// fixed.  12,288-site water, no skin: 239 -> 111 us, 3,009 sites at a 2.5 A
+// skin 92 -> 54 us, the adjoint of 16 x 1024 Wolf waters 1203 -> 646 us, of
+// which the VALU is busy 58% (the rest is load latency: 128 registers, four
+// waves per SIMD).  LJ pairs have a queue of their own: with charges on every site
+// they are few (1 in 9 in three-site water), and their code would run in
+// every evaluation for them.  The next evaluation's positions are loaded
+// before the current one's terms are computed.
+constexpr int PQ = 32;  // queue entries per atom (a trigger leaves 8 free)
+
+template <int ELEC, bool GRAD, int WPC>
+__global__ void __launch_bounds__(64 * WPC, 4) k_pair(
     const int* __restrict__ ncl_total, int maxcl, const RepDev* __restrict__ reps,
     const SiteDev* __restrict__ sites, const double4* __restrict__ cl_center,
     const float4* __restrict__ cl_box, const float4* __restrict__ plist,
     const int* __restrict__ plist_n, int cap, const int* __restrict__ slot_orig,
     const int2* __restrict__ slot_info, const double4* __restrict__ slot_x64,
-    const float4* __restrict__ slot_off,
+    const float4* __restrict__ slot_off, const float4* __restrict__ slot_par,
     double* __restrict__ fx, double* __restrict__ fy, double* __restrict__ fz,
     double* __restrict__ epart, unsigned long long* __restrict__ ipart, int want_hash,
     double* __restrict__ gq, double* __restrict__ ge, double* __restrict__ gs) {
-    static_assert(FP64, "the mixed-precision path is k_pair_mx");
+    constexpr bool EL = ELEC != 0;
     __shared__ double sh_f[WPC][MSPMS_CL][6];
     __shared__ double sh_e[WPC][4];
     __shared__ unsigned long long sh_n[WPC][4];
+    __shared__ int sh_q[WPC][EL ? 2 : 1][MSPMS_CL][PQ];
     const int ci = xcd_block(blockIdx.x, gridDim.x);
-    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    // (uniform for the compiler too: the entry loop then runs on scalars)
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int ncl = min(*ncl_total, maxcl);
     if (ci >= ncl) return;  // whole workgroup
     const int isub = lane >> 3, jsub = lane & 7;
 
     const double4 Ci = cl_center[ci];
-    const RepDev& R = reps[(int)Ci.w];
+    // (uniform: the replica's constants then sit in scalar registers)
+    const RepDev& R = reps[__builtin_amdgcn_readfirstlane((int)Ci.w)];
     const int islot = ci * MSPMS_CL + isub;
     const int2 infoi = slot_info[islot];
+    const float4 pi4f = slot_off[islot];
+    const float4 qi4f = slot_par[islot];
+    const double4 pi4 = slot_x64[islot];
+    const int moli = __float_as_int(qi4f.z), fli = __float_as_int(qi4f.w);
     const bool vi = infoi.y >= 0;
     const int oi = slot_orig[islot];
-    SiteDev si;
-    if (vi) si = sites[infoi.y];
-    const bool lji = vi && si.ghost != MSPMS_GHOST_LJ;
+    const double Cqi = vi ? R.C * pi4.w : 0.0;
+    const int atom0 = R.atom0;
 
     double afx = 0.0, afy = 0.0, afz = 0.0;
     double g_q = 0.0, g_e = 0.0, g_s = 0.0;  // d(pair energy)/d(own q, eps, sigma)
     double e_lj = 0.0, e_sh = 0.0, e_re = 0.0, vir = 0.0;
-    unsigned long long n_lj = 0, n_el = 0, h_lj = 0, h_el = 0;
+    unsigned int n_lj = 0, n_el = 0;
+    unsigned long long h_lj = 0, h_el = 0;
 
-    const int nrow = plist_n[ci];
-    const float4* row = plist + (size_t)ci * cap;
+    // the reference's separation: d - L rint(d / L).  rint(d / L) is taken
+    // from d times 1 / L unless that lies within 1e-7 of a half, where the
+    // two could round to different integers.
+    auto mic = [](double d, double L, double iL) {
+#pragma clang fp contract(off)
+        const double t = d * iL;
+        double n = rint(t);
+        if (!(fabs(t - n) <= 0.4999999)) n = rint(d / L);
+        return d - L * n;
+    };
+    struct Batch {
+        double4 p;
+        int o, slot;
+        bool on;
+    };
+    auto separate = [&](const Batch& B, double& rx, double& ry, double& rz) {
+#pragma clang fp contract(off)
+        rx = mic(pi4.x - B.p.x, R.L[0], R.invL[0]);
+        ry = mic(pi4.y - B.p.y, R.L[1], R.invL[1]);
+        rz = mic(pi4.z - B.p.z, R.L[2], R.invL[2]);
+        return rx * rx + ry * ry + rz * rz;
+    };
+    auto eval_el = [&](const Batch& B) {
+        double rx, ry, rz;
+        const double rsq = separate(B, rx, ry, rz);
+        if (!(B.on && rsq < R.rc2_el)) return;
+        const double ri = rsqrt_fma(rsq), r = rsq * ri, x = R.kappa * r;
+        double ex;
+        const double ec = erfc_exp64(x, &ex);
+        const double cq = Cqi * B.p.w;
+        double ug, f;  // energy per charge product, force / r
+        if (ELEC == MSPMS_ELEC_EWALD) {
+            ug = ri * ec;
+            f = cq * fma(ri * x * ex, 1.1283791670955126, ug) * (ri * ri);
+        } else {
+            ug = fma(ec, ri, fma(R.wvc2, r - R.rc_el, R.wvc1));
+            f = cq * ri * (fma(ec, ri, R.wfc1 * ex) * ri + R.wfc2);
+            vir += f * rsq;
+        }
+        e_re += cq * ug;
+        // the pair energy is linear in q_i: du/dq_i = u(q_i = 1)
+        if (GRAD) g_q += R.C * B.p.w * ug;
+        afx += f * rx;
+        afy += f * ry;
+        afz += f * rz;
+        if (oi < B.o) {
+            n_el++;
+            if (want_hash) h_el += pair_key(oi - atom0, B.o - atom0);
+        }
+    };
+    auto eval_lj = [&](const Batch& B) {
+        double rx, ry, rz;
+        const double rsq = separate(B, rx, ry, rz);
+        if (!(B.on && rsq < R.rc2_lj)) return;
+        const SiteDev &si = sites[infoi.y], &sj = sites[slot_info[B.slot].y];
+        const double sje = sj.epsilon;
+        double u, f, ush, sij, eij;
+        {
+#pragma clang fp contract(off)
+            sij = 0.5 * (si.sigma + sj.sigma);
+            eij = sqrt(si.epsilon * sje);
+        }
+        lj64(rsq, sij, eij, R.switch_on, R.rc2_lj, R.rcon2, R.roff2_ron2_cube, R.shift1, &u, &f,
+             &ush);
+        e_lj += u;
+        e_sh += ush;
+        vir += f * rsq;
+        if (GRAD) {
+            double dds, dde;
+            lj64_dparam(rsq, sij, eij, R.switch_on, R.rc2_lj, R.rcon2, R.roff2_ron2_cube, &dds,
+                        &dde);
+            g_s += 0.5 * dds;  // d sigma_ij / d sigma_i = 1/2
+            g_e += dde * deps_mix(eij, sje);
+        }
+        afx += f * rx;
+        afy += f * ry;
+        afz += f * rz;
+        if (oi < B.o) {
+            n_lj++;
+            if (want_hash) h_lj += pair_key(oi - atom0, B.o - atom0);
+        }
+    };
 
-    // row pruning as in k_pair_mx: an entry whose current cluster boxes are
-    // farther apart than the cutoff (with a margin of 1e-3 of it above FP32
-    // rounding) holds no pair in range; the test is the same for every lane
-    // of the wave, and the pairs that interact are still decided per pair
+    // the queues: of atom isub, entries hd .. hd + cn - 1 (modulo PQ)
+    int hd[2] = {0, 0}, cn[2] = {0, 0};
+    constexpr int QL = EL ? 1 : 0;  // the LJ queue
+    auto push = [&](int k, bool hit, int jslot) {
+        const int grp = (int)(__ballot(hit) >> (8 * isub)) & 0xff;
+        if (hit)
+            sh_q[w][k][isub][(hd[k] + cn[k] + __popc(grp & ((1 << jsub) - 1))) & (PQ - 1)] = jslot;
+        cn[k] += __popc(grp);
+    };
+    auto pop = [&](int k) {
+        Batch B;
+        B.on = jsub < cn[k];
+        __builtin_amdgcn_wave_barrier();
+        B.slot = B.on ? sh_q[w][k][isub][(hd[k] + jsub) & (PQ - 1)] : islot;
+        const int n = min(cn[k], 8);
+        hd[k] += n;
+        cn[k] -= n;
+        B.p = slot_x64[B.slot];
+        B.o = slot_orig[B.slot];
+        return B;
+    };
+    // row pruning as in k_pair_mx
     const float rprune = (float)fmax(R.rc_lj, R.rc_el) * 1.001f;
     const float rprune2 = rprune * rprune;
     const float4 bim = cl_box[2 * ci], bih = cl_box[2 * ci + 1];
-    {
-        const double4 pi4 = slot_x64[islot];
-        for (int e = w; e < nrow; e += WPC) {
-            const float4 E = row[e];
-            const uint32_t ent = __float_as_uint(E.w);
+    const float Lx = (float)R.L[0], Ly = (float)R.L[1], Lz = (float)R.L[2];
+    const float iLx = (float)R.invL[0], iLy = (float)R.invL[1], iLz = (float)R.invL[2];
+    // the first test's radii: the FP32 separation is a sum of three numbers
+    // below about 1.5 L, off by less than 1e-6 L
+    const float slack = 1e-6f * fmaxf(Lx, fmaxf(Ly, Lz));
+    const float tlj = (float)R.rc_lj * 1.0005f + slack, tel = (float)R.rc_el * 1.0005f + slack;
+    const float t2lj = tlj * tlj, t2el = tel * tel;
+
+    const int nrow = plist_n[ci];
+    const float4* row = plist + (size_t)ci * cap;
+    const int nmine = nrow > w ? (nrow - w + WPC - 1) / WPC : 0;
+    // this wave's entries, 64 at a time (one per lane), pruned, and visited
+    // in row order; an entry's j data are loaded one entry before their use
+    struct JSet {
+        float4 sep, pj, qj;
+    };
+    float4 my_ent = make_float4(0.f, 0.f, 0.f, 0.f);
+    uint64_t kept = 0;
+    int base = -64;
+    auto next = [&](JSet& J) {
+        while (kept == 0) {
+            base += 64;
+            if (base >= nmine) return false;
+            bool keep = base + lane < nmine;
+            my_ent = keep ? row[w + (base + lane) * WPC] : make_float4(0.f, 0.f, 0.f, 0.f);
+            const uint32_t ent = __float_as_uint(my_ent.w);
             const int cj = (int)(ent >> 7);
-            if (cj != ci && !(ent & 64u)) {
+            if (keep && cj != ci && !(ent & 64u)) {
                 const float4 bjm = cl_box[2 * cj], bjh = cl_box[2 * cj + 1];
-                const float gx = fmaxf(fabsf(E.x + (bim.x - bjm.x)) - (bih.x + bjh.x), 0.f);
-                const float gy = fmaxf(fabsf(E.y + (bim.y - bjm.y)) - (bih.y + bjh.y), 0.f);
-                const float gz = fmaxf(fabsf(E.z + (bim.z - bjm.z)) - (bih.z + bjh.z), 0.f);
-                if (!(gx * gx + gy * gy + gz * gz < rprune2)) continue;
+                const float gx = fmaxf(fabsf(my_ent.x + (bim.x - bjm.x)) - (bih.x + bjh.x), 0.f);
+                const float gy = fmaxf(fabsf(my_ent.y + (bim.y - bjm.y)) - (bih.y + bjh.y), 0.f);
+                const float gz = fmaxf(fabsf(my_ent.z + (bim.z - bjm.z)) - (bih.z + bjh.z), 0.f);
+                keep = gx * gx + gy * gy + gz * gz < rprune2;
             }
-            const int jslot = cj * MSPMS_CL + jsub;
-            const int2 infoj = slot_info[jslot];
-            if (!(vi && infoj.y >= 0 && infoj.x != infoi.x)) continue;
-            const double4 pj4 = slot_x64[jslot];
-            double rx, ry, rz, rsq;
-            {
-#pragma clang fp contract(off)
-                rx = pi4.x - pj4.x;
-                ry = pi4.y - pj4.y;
-                rz = pi4.z - pj4.z;
-                rx = rx - R.L[0] * rint(rx / R.L[0]);
-                ry = ry - R.L[1] * rint(ry / R.L[1]);
-                rz = rz - R.L[2] * rint(rz / R.L[2]);
-                rsq = rx * rx + ry * ry + rz * rz;
-            }
-            const SiteDev sj = sites[infoj.y];
-            const int oj = slot_orig[jslot];
-            const bool count = oi < oj;
-            if (lji && sj.ghost != MSPMS_GHOST_LJ && rsq < R.rc2_lj) {
-                double u, f, ush;
-                double sij, eij;
-                {
-#pragma clang fp contract(off)
-                    sij = 0.5 * (si.sigma + sj.sigma);
-                    eij = sqrt(si.epsilon * sj.epsilon);
-                }
-                lj64(rsq, sij, eij, R.switch_on, R.rc2_lj, R.rcon2, R.roff2_ron2_cube, R.shift1,
-                     &u, &f, &ush);
-                e_lj += u;
-                e_sh += ush;
-                vir += f * rsq;
-                if (GRAD) {
-                    double dds, dde;
-                    lj64_dparam(rsq, sij, eij, R.switch_on, R.rc2_lj, R.rcon2, R.roff2_ron2_cube,
-                                &dds, &dde);
-                    g_s += 0.5 * dds;  // d sigma_ij / d sigma_i = 1/2
-                    g_e += dde * deps_mix(eij, sj.epsilon);
-                }
-                afx += f * rx;
-                afy += f * ry;
-                afz += f * rz;
-                if (count) {
-                    n_lj++;
-                    if (want_hash) h_lj += pair_key(oi - R.atom0, oj - R.atom0);
-                }
-            }
-            if (ELEC != 0 && rsq < R.rc2_el) {
-                double u, f;
-                double qq;
-                {
-#pragma clang fp contract(off)
-                    qq = si.charge * sj.charge;
-                }
-                if (ELEC == MSPMS_ELEC_EWALD) {
-                    ewald_real64(rsq, qq, R.C, R.kappa, &u, &f);
-                } else {
-                    wolf_real64(rsq, qq, R.C, R.kappa, R.rc_el, R.wvc1, R.wvc2, R.wfc1, R.wfc2, &u,
-                                &f);
-                    vir += f * rsq;
-                }
-                e_re += u;
-                if (GRAD) {
-                    // the pair energy is linear in q_i: du/dq_i = u(q_i = 1)
-                    double ug, fg;
-                    if (ELEC == MSPMS_ELEC_EWALD)
-                        ewald_real64(rsq, sj.charge, R.C, R.kappa, &ug, &fg);
-                    else
-                        wolf_real64(rsq, sj.charge, R.C, R.kappa, R.rc_el, R.wvc1, R.wvc2, R.wfc1,
-                                    R.wfc2, &ug, &fg);
-                    g_q += ug;
-                }
-                afx += f * rx;
-                afy += f * ry;
-                afz += f * rz;
-                if (count) {
-                    n_el++;
-                    if (want_hash) h_el += pair_key(oi - R.atom0, oj - R.atom0);
-                }
-            }
+            kept = __ballot(keep);
         }
+        const int k = __builtin_ctzll(kept);
+        kept &= kept - 1;
+        J.sep = make_float4(
+            __int_as_float(__builtin_amdgcn_readlane(__float_as_int(my_ent.x), k)),
+            __int_as_float(__builtin_amdgcn_readlane(__float_as_int(my_ent.y), k)),
+            __int_as_float(__builtin_amdgcn_readlane(__float_as_int(my_ent.z), k)),
+            __int_as_float(__builtin_amdgcn_readlane(__float_as_int(my_ent.w), k)));
+        const int cj = (int)(__float_as_uint(J.sep.w) >> 7);
+        J.pj = slot_off[cj * MSPMS_CL + jsub];
+        J.qj = slot_par[cj * MSPMS_CL + jsub];
+        return true;
+    };
+    Batch be{}, bl{};
+    bool have_e = false, have_l = false;
+    JSet A;
+    bool more = next(A);
+    // one place for each evaluation, so that its constants are held once:
+    // after the entries, the turns go on until the queues are empty
+    for (;;) {
+        if (more) {
+            const JSet J = A;
+            more = next(A);
+            const uint32_t ent = __float_as_uint(J.sep.w);
+            const int jslot = (int)(ent >> 7) * MSPMS_CL + jsub;
+            const int flj = __float_as_int(J.qj.w);
+            float rx = J.sep.x + (pi4f.x - J.pj.x);
+            float ry = J.sep.y + (pi4f.y - J.pj.y);
+            float rz = J.sep.z + (pi4f.z - J.pj.z);
+            if (ent & 64u) {
+                rx -= Lx * rintf(rx * iLx);
+                ry -= Ly * rintf(ry * iLy);
+                rz -= Lz * rintf(rz * iLz);
+            }
+            const float rsq = rx * rx + ry * ry + rz * rz;
+            const bool act = vi && (flj & SLOT_VALID) && __float_as_int(J.qj.z) != moli;
+            if (EL) push(0, act && rsq < t2el, jslot);
+            push(QL, act && rsq < t2lj && (fli & flj & SLOT_LJ), jslot);
+        }
+        const int full = more ? PQ - 8 : 0;
+        const bool te = EL && (__ballot(cn[0] > full) != 0 || (!more && have_e));
+        const bool tl = __ballot(cn[QL] > full) != 0 || (!more && have_l);
+        if (te) {
+            const bool any = __ballot(cn[0] > 0) != 0;
+            const Batch n = pop(0);
+            if (have_e) eval_el(be);
+            be = n;
+            have_e = any;
+        }
+        if (tl) {
+            const bool any = __ballot(cn[QL] > 0) != 0;
+            const Batch n = pop(QL);
+            if (have_l) eval_lj(bl);
+            bl = n;
+            have_l = any;
+        }
+        if (!more && !te && !tl) break;
     }
 
     // per-atom partials: 8 j-lanes of each i, then the WPC waves in order
@@ -628,10 +752,10 @@ template <int ELEC, bool GRAD, int WPC>
 void launch_64(const LaunchCtx& c, const ClusterBufs& b, double* fx, double* fy, double* fz,
                double* epart, unsigned long long* ipart, int want_hash, double* gq, double* ge,
                double* gs) {
-    hipLaunchKernelGGL((k_pair<ELEC, true, GRAD, WPC>), dim3((b.maxcl + 7) / 8 * 8),
-                       dim3(64 * WPC), 0, c.stream, b.ncl_total, b.maxcl, c.reps, c.sites,
-                       b.cl_center, b.cl_box, b.plist, b.plist_n, b.cap, b.slot_orig, b.slot_info,
-                       b.slot_x64, b.slot_off, fx, fy, fz, epart, ipart, want_hash, gq, ge, gs);
+    hipLaunchKernelGGL((k_pair<ELEC, GRAD, WPC>), dim3((b.maxcl + 7) / 8 * 8), dim3(64 * WPC), 0,
+                       c.stream, b.ncl_total, b.maxcl, c.reps, c.sites, b.cl_center, b.cl_box,
+                       b.plist, b.plist_n, b.cap, b.slot_orig, b.slot_info, b.slot_x64, b.slot_off,
+                       b.slot_par, fx, fy, fz, epart, ipart, want_hash, gq, ge, gs);
 }
 
 template <int ELEC, int WPC, bool HALF, bool HASH>

@@ -111,6 +111,88 @@ __host__ __device__ inline void wolf_real64(double rijsq, double qq, double C, d
                              f2);
 }
 
+// ---- FP64, shared transcendentals ------------------------------------------
+// 1 / x within an ulp: the hardware estimate and two Newton steps
+__device__ inline double rcp_nr(double x) {
+    double y = __builtin_amdgcn_rcp(x);
+    y = fma(y, fma(-x, y, 1.0), y);
+    return fma(y, fma(-x, y, 1.0), y);
+}
+
+// 1 / sqrt(x) within an ulp (infinity at 0)
+__device__ inline double rsqrt_fma(double x) {
+    const double y0 = __builtin_amdgcn_rsq(x);
+    double y = y0;
+    double h = 0.5 * x * y;
+    y = fma(y, fma(-h, y, 0.5), y);
+    h = 0.5 * x * y;
+    y = fma(y, fma(-h, y, 0.5), y);
+    return x == 0.0 ? y0 : y;
+}
+
+// erfc(x) and exp(-x^2) for x >= 0 without a branch: erfc(x) = exp(-x^2)
+// P(t) / (1 + 2 x) with t = (x - K) / (x + K), the mapping of Shepherd and
+// Laframboise (Math. Comp. 36, 1981) with K = 3.75; P is the degree-22
+// truncation of the Chebyshev series of (1 + 2 x) exp(x^2) erfc(x) in t,
+// computed with 70 digits and summed into powers of t (all coefficients
+// below 1.24, so Horner's rule loses nothing): 2.6e-16 relative on
+// [0.05, 12].  The exponential is 2^n exp(r), |r| <= ln 2 / 2, by its Taylor
+// polynomial of degree 13 (remainder 4e-18), with the rounding of x^2 taken
+// back out.  The math library's erfc branches by range, so that a wave with
+// mixed arguments runs every range, and evaluates its own exponential.
+//
+// The coefficients (highest power first, then 1 / 13! .. 1 / 2!) are read
+// through the scalar cache where they are used: as literals they would be
+// kept in 70 vector registers across the caller's loop, half of what a wave
+// has at four waves per SIMD.
+constexpr int ERFC_NP = 23, ERFC_NE = 12;
+__device__ __constant__ const double erfc_coef[ERFC_NP + ERFC_NE] = {
+    -2.623107347133476e-09, -1.9551358868985616e-09, 3.197926671666804e-08,
+    1.879082322370048e-08, -2.4857126248016745e-07, -5.084465378687302e-08,
+    1.7419821586224816e-06, -9.792625707303523e-07, -1.1438048033346894e-05,
+    2.2387565714911816e-05, 5.164652974177416e-05, -0.00029015535246077655,
+    0.000293714378044958, 0.0017556261651970652, -0.009746579683265262,
+    0.02836227737211114, -0.05869339857664934, 0.09230432116428125,
+    -0.10880393014244462, 0.08227673848999506, 0.0035854154854790257,
+    -0.14024059858554525, 1.2375126308378275,
+    1.6059043836821613e-10, 2.08767569878681e-09, 2.505210838544172e-08,
+    2.755731922398589e-07, 2.7557319223985893e-06, 2.48015873015873e-05,
+    0.0001984126984126984, 0.001388888888888889, 0.008333333333333333,
+    0.041666666666666664, 0.16666666666666666, 0.5};
+typedef const double __attribute__((address_space(4))) scalar_double;
+
+// a b + c with c in scalar registers (the compiler's own choice, the
+// two-operand form, first copies c into vector registers: as many cycles as
+// the multiply-add)
+__device__ inline double fma_sc(double a, double b, double c) {
+    double d;
+    asm("v_fma_f64 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "s"(c));
+    return d;
+}
+
+__device__ inline double erfc_exp64(double x, double* ex) {
+    scalar_double* c = (scalar_double*)erfc_coef;
+    asm volatile("" : "+s"(c));  // loaded here, not ahead of the caller's loop
+    const double s = x * x;
+    // exp(-s)
+    const double n = rint(s * -1.4426950408889634);
+    double r = fma(n, -0x1.62e42fefa39efp-1, -s);
+    r = fma(n, -0x1.abc9e3b39803fp-56, r);
+    double e = c[ERFC_NP];
+#pragma unroll
+    for (int k = 1; k < ERFC_NE; k++) e = fma_sc(e, r, c[ERFC_NP + k]);
+    e = ldexp(fma(e * r, r, r) + 1.0, (int)n);
+    e = fma(-fma(x, x, -s), e, e);
+    const double a = x + 3.75, b = fma(2.0, x, 1.0);
+    const double q = rcp_nr(a * b);
+    const double t = (x - 3.75) * (q * b);
+    double p = c[0];
+#pragma unroll
+    for (int k = 1; k < ERFC_NP; k++) p = fma_sc(p, t, c[k]);
+    *ex = e;
+    return e * (p * (q * a));
+}
+
 // ---- FP32 ---------------------------------------------------------------
 // erfc(x) = exp(-x^2) * P(t), t = 1/(1 + x/2), x >= 0.  P is a degree-9
 // weighted least-squares fit of the scaled complementary error function
