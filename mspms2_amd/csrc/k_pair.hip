@@ -52,6 +52,11 @@ __device__ inline float dpp_f32(float v) {
     return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xF, 0xF, true));
 }
 
+// an FP32 constant of the whole wave in a scalar register
+__device__ inline float uni(double v) {
+    return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int((float)v)));
+}
+
 // XCD-aware block order: consecutive i-clusters (spatial neighbours that
 // share j-clusters) land on the same XCD and its L2.
 __device__ inline int xcd_block(int b, int nb) {
@@ -417,13 +422,15 @@ __global__ void __launch_bounds__(64 * WPC) k_pair_mx(
     const int ci = xcd_block(blockIdx.x, gridDim.x);
     const int ncl = min(*ncl_total, maxcl);
     if (ci >= ncl) return;  // whole workgroup
-    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    // (uniform for the compiler: the entry loop's control flow and the row's
+    // bookkeeping then run on scalars; 12,288-site step 91.0 -> 89.6 us)
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     // HALF: i = lane & 7, so that the eight i-lanes of a j are adjacent and
     // their per-entry sum takes three DPP steps; otherwise i = lane >> 3
     const int isub = HALF ? (lane & 7) : (lane >> 3), jsub = HALF ? (lane >> 3) : (lane & 7);
 
     const double4 Ci = cl_center[ci];
-    const RepDev& R = reps[(int)Ci.w];
+    const RepDev& R = reps[__builtin_amdgcn_readfirstlane((int)Ci.w)];
     const int islot = ci * MSPMS_CL + isub;
     const float4 pi4 = slot_off[islot];
     const float4 qi4 = slot_par[islot];
@@ -431,15 +438,15 @@ __global__ void __launch_bounds__(64 * WPC) k_pair_mx(
     const bool vi = (fli & SLOT_VALID) != 0;
     const int oi = want_hash && vi ? slot_orig[islot] - R.atom0 : 0;
     const float q_i = pi4.w;
-    const float rc2lj = (float)R.rc2_lj, rc2el = (float)R.rc2_el;
-    const float Lx = (float)R.L[0], Ly = (float)R.L[1], Lz = (float)R.L[2];
-    const float iLx = (float)R.invL[0], iLy = (float)R.invL[1], iLz = (float)R.invL[2];
-    const float kappa = (float)R.kappa, Cf = (float)R.C, shift1 = (float)R.shift1;
-    const float rcel = (float)R.rc_el, v1 = (float)R.wvc1, v2 = (float)R.wvc2,
-                f1 = (float)R.wfc1, f2 = (float)R.wfc2;
-    const float rcon2 = (float)R.rcon2, inv_den = (float)(1.0 / R.roff2_ron2_cube);
-    // replica constants in registers: a reload inside the entry loop would
-    // wait for the prefetched loads
+    const float rc2lj = uni(R.rc2_lj), rc2el = uni(R.rc2_el);
+    const float Lx = uni(R.L[0]), Ly = uni(R.L[1]), Lz = uni(R.L[2]);
+    const float iLx = uni(R.invL[0]), iLy = uni(R.invL[1]), iLz = uni(R.invL[2]);
+    const float kappa = uni(R.kappa), Cf = uni(R.C), shift1 = uni(R.shift1);
+    const float rcel = uni(R.rc_el), v1 = uni(R.wvc1), v2 = uni(R.wvc2),
+                f1 = uni(R.wfc1), f2 = uni(R.wfc2);
+    const float rcon2 = uni(R.rcon2), inv_den = uni(1.0 / R.roff2_ron2_cube);
+    // replica constants in (scalar) registers: a reload inside the entry loop
+    // would wait for the prefetched loads
     const bool sw_on = R.switch_on != 0;
     const int atom0 = R.atom0;
     // pruning of the row: an entry whose current cluster boxes are farther
