@@ -20,8 +20,10 @@
 //                 (ushift - old)] / treq; accept if dH <= 0 or a uniform
 //                 draw < exp(-dH); otherwise restore the positions; with
 //                 per-chain steps, the equilibration-phase delt adjustment
-// The random draws are sequential per replica (one lane); momentum,
-// kinetic energy and the position save / restore use the whole workgroup.
+// The velocities' random numbers are drawn by the whole workgroup
+// (draw_velocities): the same stream, in the same order, as one lane drawing
+// them in turn (2650 us of a 6600 us move of 64 butane boxes of 64-512
+// molecules; 51 us now).
 #include "engine.h"
 #include "../../include/mspms_gpu.h"
 
@@ -41,25 +43,149 @@ __device__ inline double ranmar_next(RanmarDev& r) {
     return uni;
 }
 
-// polar method, the second deviate of each accepted pair kept for the next
-// call (gaussran, src/random.c:113-138)
-__device__ inline double gaussran(RanmarDev& r) {
+// The stream in integers (every value is a multiple of 2^-24): with X_n the
+// n-th lagged value and C_n the n-th term of the arithmetic sequence,
+//     X_n = (X_{n-97} - X_{n-33}) mod 2^24,
+//     C_n = (C_0 - n cd) mod cm,    draw n = (X_n - C_n) mod 2^24.
+// 33 lanes step together: lane l's X_{n-33} is its own last value, and its
+// X_{n-97} was stored at least two rounds before.
+constexpr int RM_ONE = 1 << 24, RM_CD = 7654321, RM_CM = 16777213;
+constexpr int RM_ROUNDS = 30, RM_BLOCK = 33 * RM_ROUNDS;  // draws per block (even)
+constexpr int HMC_T = 256;                                // threads per replica
+
+struct DrawLds {
+    int x[97 + RM_BLOCK];  // X_{n-96} .. X_n, then the block's values
+    int wsum[HMC_T / 64];
+    int used, have;
+    double gset;
+};
+
+// v = sqrt(treq / m) * Gaussian for every component of every atom of the
+// replica, in atom order (the draws of velinit, src/initvars.c:151-232, by
+// the polar method of gaussran, src/random.c:113-138: pairs of draws are
+// taken until one falls inside the unit circle; its two deviates go to the
+// next two components).  The block's pairs are tested side by side, an
+// accepted pair's place in the sequence is its rank among the accepted ones,
+// and the stream is left where the last pair that was needed left it.
+__device__ void draw_velocities(const RepDev& R, double treq, RanmarDev& rng,
+                                const double* __restrict__ aw_atom, double* vx, double* vy,
+                                double* vz, DrawLds& D) {
 #pragma clang fp contract(off)
-    if (r.iset) {
-        r.iset = 0;
-        return r.gset;
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    const long ng = 3L * R.natom;
+    const double stdvtmp = sqrt(treq);
+    double* const v[3] = {vx, vy, vz};
+    auto put = [&](long k, double g) {
+        const int i = R.atom0 + (int)(k / 3);
+        v[k % 3][i] = (stdvtmp / sqrt(aw_atom[i])) * g;
+    };
+    const int i97 = rng.i97, j97 = rng.j97, iset = rng.iset;
+    const int c0 = (int)(rng.c * RM_ONE);
+    if (ng == 0) return;  // uniform
+    if (iset && t == 0) put(0, rng.gset);
+    const long need = ng - (iset ? 1 : 0), npair = (need + 1) / 2;
+    // slot ((i97 - 1 + k) mod 97) + 1 holds the value of k draws ago
+    for (int k = 1 + t; k <= 97; k += HMC_T) D.x[97 - k] = (int)(rng.u[(i97 - 1 + k) % 97 + 1] * RM_ONE);
+    long done = 0, total = 0;  // pairs accepted, draws taken, before the block
+    int used = 0;              // draws of the block that were needed
+    for (;;) {
+        __syncthreads();
+        if (w == 0 && lane < 33) {
+            int prev = D.x[64 + lane];
+            for (int r = 0; r < RM_ROUNDS; r++) {
+                const int n = 33 * r + lane;
+                prev = (*(volatile int*)&D.x[n] - prev) & (RM_ONE - 1);
+                *(volatile int*)&D.x[97 + n] = prev;
+                __builtin_amdgcn_wave_barrier();
+            }
+        }
+        if (t == 0) {
+            D.used = RM_BLOCK;
+            D.have = 0;
+        }
+        __syncthreads();
+        // thread t: pairs 2 t and 2 t + 1 (draws 4 t .. 4 t + 3)
+        double rsq[2] = {0.0, 0.0}, v1[2], v2[2];
+        bool ok[2] = {false, false};
+        int cnt = 0;
+        if (4 * t < RM_BLOCK) {
+            long cl = ((long)c0 - (total + 4 * t + 1) * RM_CD) % RM_CM;
+            int cc = (int)(cl < 0 ? cl + RM_CM : cl);
+            double u[4];
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const int x = 4 * t + k < RM_BLOCK ? D.x[97 + 4 * t + k] : 0;
+                u[k] = ((x - cc) & (RM_ONE - 1)) * (1.0 / RM_ONE);
+                cc -= RM_CD;
+                if (cc < 0) cc += RM_CM;
+            }
+#pragma unroll
+            for (int k = 0; k < 2; k++) {
+                v1[k] = 2.0 * u[2 * k] - 1.0;
+                v2[k] = 2.0 * u[2 * k + 1] - 1.0;
+                rsq[k] = v1[k] * v1[k] + v2[k] * v2[k];
+                ok[k] = 4 * t + 2 * k < RM_BLOCK && !(rsq[k] >= 1.0 || rsq[k] == 0.0);
+                cnt += ok[k] ? 1 : 0;
+            }
+        }
+        // this thread's first rank: the accepted pairs of the threads before it
+        int incl = cnt;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int q = __shfl_up(incl, o, 64);
+            if (lane >= o) incl += q;
+        }
+        if (lane == 63) D.wsum[w] = incl;
+        __syncthreads();
+        long rank = done + incl - cnt;
+        int all = 0;
+        for (int k = 0; k < HMC_T / 64; k++) {
+            if (k < w) rank += D.wsum[k];
+            all += D.wsum[k];
+        }
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            if (!ok[k]) continue;
+            if (rank < npair) {
+                const double fac = sqrt(-2.0 * log(rsq[k]) / rsq[k]);
+                const long g = 2 * rank;
+                put(g + (iset ? 1 : 0), v2[k] * fac);
+                if (g + 1 < need)
+                    put(g + 1 + (iset ? 1 : 0), v1[k] * fac);
+                else {
+                    D.gset = v1[k] * fac;
+                    D.have = 1;
+                }
+                if (rank == npair - 1) D.used = 4 * t + 2 * k + 2;
+            }
+            rank++;
+        }
+        __syncthreads();
+        done += all;
+        used = D.used;
+        total += used;
+        if (done >= npair) break;
+        // the last 97 values open the next block
+        int keep[1 + 97 / HMC_T];
+        for (int k = t, q = 0; k < 97; k += HMC_T, q++) keep[q] = D.x[RM_BLOCK + k];
+        __syncthreads();
+        for (int k = t, q = 0; k < 97; k += HMC_T, q++) D.x[k] = keep[q];
     }
-    double v1, v2, rsq;
-    do {
-        const double a = ranmar_next(r), b = ranmar_next(r);
-        v1 = 2.0 * a - 1.0;
-        v2 = 2.0 * b - 1.0;
-        rsq = v1 * v1 + v2 * v2;
-    } while (rsq >= 1.0 || rsq == 0.0);
-    const double fac = sqrt(-2.0 * log(rsq) / rsq);
-    r.gset = v1 * fac;
-    r.iset = 1;
-    return v2 * fac;
+    // the generator after `total` draws: both cursors step down through 97..1
+    const int ni = (int)(((i97 - 1 - total) % 97 + 97) % 97) + 1;
+    const int nj = (int)(((j97 - 1 - total) % 97 + 97) % 97) + 1;
+    __syncthreads();
+    for (int k = 1 + t; k <= 97; k += HMC_T)
+        rng.u[(ni - 1 + k) % 97 + 1] = D.x[used + 97 - k] * (1.0 / RM_ONE);
+    if (t == 0) {
+        rng.i97 = ni;
+        rng.j97 = nj;
+        const long cl = ((long)c0 - total * RM_CD) % RM_CM;
+        rng.c = (cl < 0 ? cl + RM_CM : cl) * (1.0 / RM_ONE);
+        rng.iset = D.have;
+        if (D.have) rng.gset = D.gset;
+    }
+    __syncthreads();
 }
 
 template <int NV>
@@ -81,21 +207,12 @@ __device__ void block_sum_hmc(double (&v)[NV], double* sh, double* out) {
     __syncthreads();
 }
 
-// velinit (src/initvars.c:151-232) for one replica: lane 0 draws, the
-// workgroup reduces and rescales
+// velinit (src/initvars.c:151-232) for one replica
 __device__ void velinit_rep(const RepDev& R, HmcRep& H, RanmarDev& rng, const double* aw_atom,
-                            double* vx, double* vy, double* vz, double* sh, double* red) {
+                            double* vx, double* vy, double* vz, double* sh, double* red,
+                            DrawLds& D) {
 #pragma clang fp contract(off)
-    if (threadIdx.x == 0) {
-        const double stdvtmp = sqrt(H.treq);
-        for (int i = R.atom0; i < R.atom0 + R.natom; i++) {
-            const double stdv = stdvtmp / sqrt(aw_atom[i]);
-            vx[i] = stdv * gaussran(rng);
-            vy[i] = stdv * gaussran(rng);
-            vz[i] = stdv * gaussran(rng);
-        }
-    }
-    __syncthreads();
+    draw_velocities(R, H.treq, rng, aw_atom, vx, vy, vz, D);
     double p[3] = {0.0, 0.0, 0.0};
     for (int i = R.atom0 + threadIdx.x; i < R.atom0 + R.natom; i += blockDim.x) {
         p[0] += vx[i] * aw_atom[i];
@@ -128,7 +245,7 @@ __device__ void velinit_rep(const RepDev& R, HmcRep& H, RanmarDev& rng, const do
 
 // start-up: velinit of every replica (the reference's init_vars draws the
 // initial velocities from the freshly seeded stream)
-__global__ void __launch_bounds__(256) k_hmc_init(const RepDev* __restrict__ reps,
+__global__ void __launch_bounds__(HMC_T) k_hmc_init(const RepDev* __restrict__ reps,
                                                   HmcRep* __restrict__ hmc,
                                                   RanmarDev* __restrict__ rng,
                                                   const double* __restrict__ aw_atom,
@@ -137,18 +254,19 @@ __global__ void __launch_bounds__(256) k_hmc_init(const RepDev* __restrict__ rep
     __shared__ double sh[4 * 4];
     __shared__ double red[4];
     __shared__ RanmarDev r;
+    __shared__ DrawLds D;
     const int rep = blockIdx.x;
     if (active && !active[rep]) return;  // whole workgroup
     if (threadIdx.x == 0) r = rng[rep];
     __syncthreads();
-    velinit_rep(reps[rep], hmc[rep], r, aw_atom, vx, vy, vz, sh, red);
+    velinit_rep(reps[rep], hmc[rep], r, aw_atom, vx, vy, vz, sh, red, D);
     if (threadIdx.x == 0) {
         rng[rep] = r;
         hmc[rep].first = 1;
     }
 }
 
-__global__ void __launch_bounds__(256) k_hmc_begin(const RepDev* __restrict__ reps,
+__global__ void __launch_bounds__(HMC_T) k_hmc_begin(const RepDev* __restrict__ reps,
                                                    HmcRep* __restrict__ hmc,
                                                    RanmarDev* __restrict__ rng,
                                                    const double* __restrict__ aw_atom,
@@ -158,6 +276,7 @@ __global__ void __launch_bounds__(256) k_hmc_begin(const RepDev* __restrict__ re
     __shared__ double sh[4 * 4];
     __shared__ double red[4];
     __shared__ RanmarDev r;
+    __shared__ DrawLds D;
     const int rep = blockIdx.x;
     const RepDev& R = reps[rep];
     HmcRep& H = hmc[rep];
@@ -167,7 +286,7 @@ __global__ void __launch_bounds__(256) k_hmc_begin(const RepDev* __restrict__ re
         (void)ranmar_next(r);  // the move-type draw of hmc() (src/hmc.c:25)
     }
     __syncthreads();
-    if (!first) velinit_rep(R, H, r, aw_atom, vx, vy, vz, sh, red);
+    if (!first) velinit_rep(R, H, r, aw_atom, vx, vy, vz, sh, red, D);
     const size_t n = (size_t)natom_total;
     for (int i = R.atom0 + threadIdx.x; i < R.atom0 + R.natom; i += blockDim.x)
         for (int d = 0; d < 3; d++) pos_old[d * n + i] = pos[d * n + i];
@@ -258,14 +377,14 @@ __global__ void k_hmc_draw(RanmarDev* rng, int rep, int n, double* out) {
 void launch_hmc_init(const LaunchCtx& c, HmcRep* hmc, RanmarDev* rng, const double* aw_atom,
                      double* vel, const int* active) {
     const size_t n = (size_t)c.natom;
-    hipLaunchKernelGGL(k_hmc_init, dim3(c.nrep), dim3(256), 0, c.stream, c.reps, hmc, rng,
+    hipLaunchKernelGGL(k_hmc_init, dim3(c.nrep), dim3(HMC_T), 0, c.stream, c.reps, hmc, rng,
                        aw_atom, vel, vel + n, vel + 2 * n, active);
 }
 
 void launch_hmc_begin(const LaunchCtx& c, HmcRep* hmc, RanmarDev* rng, const double* aw_atom,
                       const double* pos, double* pos_old, double* vel) {
     const size_t n = (size_t)c.natom;
-    hipLaunchKernelGGL(k_hmc_begin, dim3(c.nrep), dim3(256), 0, c.stream, c.reps, hmc, rng,
+    hipLaunchKernelGGL(k_hmc_begin, dim3(c.nrep), dim3(HMC_T), 0, c.stream, c.reps, hmc, rng,
                        aw_atom, pos, pos_old, vel, vel + n, vel + 2 * n, c.natom);
 }
 
