@@ -12,9 +12,7 @@
 // and, only when a rebuild is requested (the others return at once):
 //   k_bin_scan per atom: wrap into the box, integer cell (cx,cy,cz), count;
 //              the last workgroup: exclusive scans over cells and columns
-//              (cells of a column are contiguous, ordered by cz); grids of
-//              more than 16,384 cells: k_scan, one workgroup of 1024
-//              threads, does the scans
+//              (cells of a column are contiguous, ordered by cz)
 //   k_scatter  per atom: cell member lists
 //   k_place_bbox  one workgroup per column: exact rank of each atom inside
 //              its cell by (wrapped z, index) -> slot in its column (a column
@@ -301,7 +299,8 @@ __device__ void scan_cells(int ncell, int ncol, int* __restrict__ cell_count,
 // Per atom: wrap into the box, integer cell, count (bin_atom).  The last
 // workgroup to finish (arrival count) scans the cells and columns
 // (scan_cells): one launch instead of two.
-__global__ void __launch_bounds__(256) k_bin_scan(
+template <int NT>
+__global__ void __launch_bounds__(NT) k_bin_scan(
     int natom, const double* __restrict__ x, const double* __restrict__ y,
     const double* __restrict__ z, const int* __restrict__ atom_site,
     const int* __restrict__ atom_mol, const SiteDev* __restrict__ sites,
@@ -316,36 +315,24 @@ __global__ void __launch_bounds__(256) k_bin_scan(
     if (i < natom)
         bin_atom(i, x, y, z, atom_site, atom_mol, sites, mols, reps, atom_cell, atom_slot, atom_wz,
                  cell_count, fx, fy, fz, atom_gslot, st);
-    if (!ctr) return;  // the cells are scanned by k_scan
     // arrival: this workgroup's counts are visible device-wide before its
-    // count
+    // arrival count.  One thread's acquire-release operation covers the
+    // workgroup's writes, which the barrier orders before it: a fence by every
+    // thread has each wave write back the XCD's L2 (70,508 atoms, 256
+    // threads: 47.7 us with it, 34.3 without; 1024 threads: 43.9 and 24.7).
     __shared__ int last;
     __shared__ int sh[32];
-    __shared__ int stage[SCAN_LDS<256>];
-    __threadfence();
+    __shared__ int stage[SCAN_LDS<NT>];
     __syncthreads();
-    if (threadIdx.x == 0) last = atomicAdd(ctr, 1) == (int)gridDim.x - 1;
+    if (threadIdx.x == 0) {
+        last = __hip_atomic_fetch_add(ctr, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) ==
+               (int)gridDim.x - 1;
+        if (last) *ctr = 0;  // for the next build
+    }
     __syncthreads();
     if (!last) return;
-    __threadfence();
-    if (threadIdx.x == 0) *ctr = 0;  // for the next build
-    scan_cells<256>(ncell, ncol, cell_count, cell_start, col_cell0, col_cl0, cl_col, ncl_total,
-                    maxcl, st, sh, stage);
-}
-
-// The cell and column scans by one workgroup of 1024 threads, for grids of
-// many cells (a workgroup of 256 at the end of k_bin_scan would take long).
-__global__ void __launch_bounds__(1024) k_scan(int ncell, int ncol, int* cell_count,
-                                               int* __restrict__ cell_start,
-                                               const int* __restrict__ col_cell0,
-                                               int* __restrict__ col_cl0, int* __restrict__ cl_col,
-                                               int* __restrict__ ncl_total, int maxcl, Status* st,
-                                               const int* lstate) {
-    if (!lstate[LS_NEED]) return;
-    __shared__ int sh[32];
-    __shared__ int stage[SCAN_LDS<1024>];
-    scan_cells<1024>(ncell, ncol, cell_count, cell_start, col_cell0, col_cl0, cl_col, ncl_total,
-                     maxcl, st, sh, stage);
+    scan_cells<NT>(ncell, ncol, cell_count, cell_start, col_cell0, col_cl0, cl_col, ncl_total,
+                   maxcl, st, sh, stage);
 }
 
 __global__ void k_scatter(int natom, const int* __restrict__ atom_cell,
@@ -726,22 +713,31 @@ void launch_cluster_build(const LaunchCtx& c, ClusterBufs& b, const double* x, c
                        b.atom_x0, b.ncl_total, b.maxcl, b.slot_orig, b.slot_w64, b.cl_center,
                        b.slot_x64, b.slot_off, b.cl_box, b.fslot, b.lstate, half_skin2, force,
                        b.half, b.hist);
-    // up to 16,384 cells the last binning workgroup scans them (one launch
-    // less per step); larger grids take a workgroup of 1024 threads
-    const bool scan_here = b.ncell <= 16384;
-    hipLaunchKernelGGL(k_bin_scan, dim3(gA), dim3(T), 0, c.stream, c.natom, x, y, z, c.atom_site,
-                       c.atom_mol, c.sites, c.mols, c.reps, b.atom_cell, b.atom_slot, b.atom_wz,
-                       b.cell_count, fx, fy, fz, b.atom_gslot, c.status, b.lstate, b.ncell,
-                       b.ncol, b.cell_start, b.col_cell0, b.col_cl0, b.cl_col, b.ncl_total,
-                       b.maxcl, scan_here ? b.bin_ctr : nullptr);
-    if (!scan_here)
-        hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, c.stream, b.ncell, b.ncol, b.cell_count,
-                           b.cell_start, b.col_cell0, b.col_cl0, b.cl_col, b.ncl_total, b.maxcl,
-                           c.status, b.lstate);
+    // the last binning workgroup scans the cells.  1024 threads scan, and
+    // arrive, faster where there are many (8,813 cells: 24.7 against 34.3 us;
+    // 6,144: 18.3 against 25.2); at 1,331 cells both take 13.0, and smaller
+    // systems would leave CUs idle while they bin.
+    auto bin = [&](auto kernel, int nt) {
+        hipLaunchKernelGGL(kernel, dim3((c.natom + nt - 1) / nt), dim3(nt), 0, c.stream, c.natom,
+                           x, y, z, c.atom_site, c.atom_mol, c.sites, c.mols, c.reps, b.atom_cell,
+                           b.atom_slot, b.atom_wz, b.cell_count, fx, fy, fz, b.atom_gslot,
+                           c.status, b.lstate, b.ncell, b.ncol, b.cell_start, b.col_cell0,
+                           b.col_cl0, b.cl_col, b.ncl_total, b.maxcl, b.bin_ctr);
+    };
+    if (b.ncell > 2048)
+        bin(k_bin_scan<1024>, 1024);
+    else
+        bin(k_bin_scan<256>, 256);
     hipLaunchKernelGGL(k_scatter, dim3(gA), dim3(T), 0, c.stream, c.natom, b.atom_cell,
                        b.atom_slot, b.cell_start, b.cell_members, b.lstate);
-    // 1024 threads: a column of a long box holds thousands of atoms
-    hipLaunchKernelGGL(k_place_bbox, dim3(b.ncol), dim3(1024), 0, c.stream, b.ncol, x, y, z,
+    // threads for 1.25 times the mean column, up to 1024 (a column of a long
+    // box holds thousands of atoms): a workgroup much larger than its column
+    // idles (70,508 atoms in 1,600 columns: 28.6 us with 1024 threads, 13.5
+    // with 64), and where no list is built it still waits for a CU with 16
+    // free waves.
+    int tp = 64;
+    while (tp < 1024 && (double)tp * b.ncol < 1.25 * c.natom) tp *= 2;
+    hipLaunchKernelGGL(k_place_bbox, dim3(b.ncol), dim3(tp), 0, c.stream, b.ncol, x, y, z,
                        b.atom_cell, b.atom_wz, b.cell_start, b.cell_members, c.atom_mol,
                        c.atom_site, c.mols, c.reps, b.col_cell0, b.col_cl0, b.col_rep,
                        b.ncl_total, b.slot_orig, b.slot_info, b.slot_x64, b.slot_w64, b.atom_x0,
