@@ -175,6 +175,7 @@ struct mspms_ctx {
     DevBuf<unsigned long long> d_fin_partu;
     DevBuf<int> d_fin_count;
     DevBuf<int> d_fin_on;    // gate of the RESPA step's finalize (1: run)
+    DevBuf<int> d_fin_off;   // a gate that stays 0 (steps whose terms nobody reads)
     DevBuf<double> d_snap;   // (6, natom) start of the last step begun
                              //   without a pair-list overflow (RESPA runs)
     DevBuf<int> d_snap_count;  // steps that wrote it since the last sync
@@ -1219,6 +1220,7 @@ int build(mspms_ctx* c) {
         (rc = c->d_fin_part.ensure((size_t)c->nrep * FIN_BLOCKS * FIN_ND)) ||
         (rc = c->d_fin_partu.ensure((size_t)c->nrep * FIN_BLOCKS * 4)) ||
         (rc = c->d_fin_count.ensure((size_t)c->nrep)) || (rc = c->d_fin_on.ensure(1)) ||
+        (rc = c->d_fin_off.ensure(1)) ||
         (rc = c->d_hist.ensure(1)) || (rc = c->d_hstep.ensure((size_t)c->nrep)) ||
         (rc = c->d_snap.ensure((size_t)6 * c->natom)) || (rc = c->d_snap_count.ensure(1)))
         return rc;
@@ -1226,6 +1228,7 @@ int build(mspms_ctx* c) {
     c->snap_pos = c->snap_vel = nullptr;
     HIPC(hipMemsetAsync(c->d_fin_count.p, 0, sizeof(int) * (size_t)c->nrep, s));
     HIPC(hipMemsetD32Async((hipDeviceptr_t)c->d_fin_on.p, 1, 1, s));
+    HIPC(hipMemsetD32Async((hipDeviceptr_t)c->d_fin_off.p, 0, 1, s));
     HIPC(hipMemsetAsync(c->d_hist.p, 0, sizeof(HistDev), s));
     HIPC(hipMemsetAsync(c->d_hstep.p, 0, sizeof(int) * (size_t)c->nrep, s));
     c->fin.part = c->d_fin_part.p;
@@ -1387,13 +1390,14 @@ __global__ void k_reset_status(Status* st) {
 
 // The frclong terms from the partial sums; with sterms, also the frcshort
 // terms of the inner steps (ep_short) and the kinetic energy (kin).
-// gated: the pass runs only while the context's finalize flag is 1 (the
-// device vver run clears it for the steps whose terms nobody reads)
+// gate (or null): the pass runs only while that flag is 1 (d_fin_on, which the
+// device vver run clears for the steps whose terms nobody reads, or d_fin_off)
 void launch_finalize(mspms_ctx* c, const LaunchCtx& L, mspms_long_terms* terms,
                      mspms_short_terms* sterms = nullptr, double* ukin = nullptr,
-                     bool gated = false, const FinAtoms* atoms = nullptr) {
+                     const int* gate = nullptr, const FinAtoms* atoms = nullptr) {
     FinBufs fb = c->fin;
-    fb.on = gated ? c->d_fin_on.p : nullptr;
+    fb.on = gate;
+    fb.off = gate && gate == c->d_fin_off.p;
     // with the wall split into the inner loop, a RESPA step (sterms) still
     // reports its energy, which the last inner step left in ep_sf; a
     // standalone frclong leaves it out
@@ -1550,10 +1554,11 @@ int enqueue_short(mspms_ctx* c, const double* x, const double* y, const double* 
 }
 
 // One RESPA velocity-Verlet outer step, NVE (src/md.c:22-83) on device
-// (3, N) SoA buffers; kernels only, so that it can be captured.
+// (3, N) SoA buffers; kernels only, so that it can be captured.  read = false:
+// nobody reads this step's terms, and their reduction is left out.
 int enqueue_vver(mspms_ctx* c, double* pos, double* vel, double* fl, double* fs, double delt,
                  int nstep_inner, mspms_long_terms* lterms, mspms_short_terms* sterms,
-                 double* ukin, hipStream_t s) {
+                 double* ukin, hipStream_t s, bool read = true) {
     const size_t n = (size_t)c->natom;
     // src/initvars.c:605-607
     const double deltby2 = delt / 2.0, delts = delt / nstep_inner, deltsby2 = delts / 2.0;
@@ -1586,11 +1591,44 @@ int enqueue_vver(mspms_ctx* c, double* pos, double* vel, double* fl, double* fs,
         // frcshort (last inner step) and kinetic terms in one pass
         ProfScope p(c, s, PROF_FINAL);
         const FinAtoms A{fl, fl + n, fl + 2 * n, c->d_frec.p, kick, c->natom, slot_forces(c)};
-        launch_finalize(c, L, lterms, sterms, ukin, true, deferred ? &A : nullptr);
+        launch_finalize(c, L, lterms, sterms, ukin, read ? c->d_fin_on.p : c->d_fin_off.p,
+                        deferred ? &A : nullptr);
     }
     HIPC(hipGetLastError());
     return 0;
 }
+
+// Steps per captured graph of a device run.  Four steps in one graph drop
+// three of the four graph boundaries per four steps (0.6 us per step at the
+// 12,288-site water step of ~97 us); the steps that four does not divide are
+// enqueued one by one, at about 16 us more each (6 NVT steps of 12,288
+// sites: 943 us as one graph of four and two steps, 910 as six graphs).  So
+// short runs take the largest count up to four that leaves none over, and
+// runs of 64 steps or more, where three such steps are made up for, take four.
+constexpr int RUN_GRAPH_STEPS = 4;
+
+int run_graph_steps(int nsteps) {
+    if (nsteps >= 16 * RUN_GRAPH_STEPS) return RUN_GRAPH_STEPS;
+    int per = RUN_GRAPH_STEPS;
+    while (per > 1 && (nsteps < per || nsteps % per)) per--;
+    return per;
+}
+
+// Closes the finalize gate for a run of device steps whose terms nobody reads
+// (written between launches, outside any capture) and opens it for the last;
+// it is open again when the run returns, whatever the path.
+struct FinGate {
+    mspms_ctx* c;
+    hipStream_t s;
+    bool closed = false;
+    hipError_t set(bool open) {
+        closed = !open;
+        return hipMemsetD32Async((hipDeviceptr_t)c->d_fin_on.p, open ? 1 : 0, 1, s);
+    }
+    ~FinGate() {
+        if (closed) (void)set(true);
+    }
+};
 
 int read_status(mspms_ctx* c, hipStream_t s) {
     HIPC(hipMemcpyAsync(c->h_status, c->d_status.p, sizeof(Status), hipMemcpyDeviceToHost, s));
@@ -1844,15 +1882,9 @@ extern "C" int mspms_vver_step_device(mspms_ctx* c, double* pos, double* vel, do
     return enqueue_vver(c, pos, vel, fl, fs, delt, nstep_inner, lterms, sterms, ukin, s);
 }
 
-// Steps per captured graph of a device run: four steps in one graph drop
-// three of the four graph boundaries per four steps (0.6 us per step at the
-// 12,288-site water step of ~97 us, A/B on one box).
-constexpr int VVER_GRAPH_STEPS = 4;
-
-// nsteps RESPA outer steps; with use_graph VVER_GRAPH_STEPS steps (one step
-// for shorter runs) are captured once as a HIP graph (on the context stream)
-// and replayed on `stream`, the last nsteps % VVER_GRAPH_STEPS steps
-// enqueued directly.  Optional histories receive each step's terms (nsteps
+// nsteps RESPA outer steps; with use_graph a few steps (run_graph_steps) are
+// captured once as a HIP graph (on the context stream) and replayed on
+// `stream`, the steps left over enqueued directly.  Optional histories receive each step's terms (nsteps
 // * nrep entries) and kinetic energies (nsteps * nrep doubles).
 extern "C" int mspms_vver_run_device(mspms_ctx* c, double* pos, double* vel, double* fl,
                                      double* fs, double delt, int nstep_inner, int nsteps,
@@ -1867,7 +1899,7 @@ extern "C" int mspms_vver_run_device(mspms_ctx* c, double* pos, double* vel, dou
     HIPC(hipSetDevice(c->device));
     hipStream_t s = stream ? (hipStream_t)stream : c->stream;
     const int nr = c->nrep;
-    const int per = nsteps >= VVER_GRAPH_STEPS ? VVER_GRAPH_STEPS : 1;
+    const int per = run_graph_steps(nsteps);
     if (use_graph) {
         mspms_ctx::GraphKey k{pos, vel, fl, fs, lterms, sterms, ukin, delt, nstep_inner, per};
         int rc = ensure_graph(c, s, GRAPH_VVER, k, [&](hipStream_t cs) {
@@ -1881,28 +1913,22 @@ extern "C" int mspms_vver_run_device(mspms_ctx* c, double* pos, double* vel, dou
         if (rc) return rc;
     }
     // without histories only the last step's terms are read: the steps
-    // before it skip the finalize pass (its gate is set between launches,
-    // outside any capture)
+    // before it skip the finalize pass
     const bool hist = lhist || shist || ukin_hist;
     const bool gate = !hist && nsteps > 1;
-    // the gate is open and the histories are off again when this call
-    // returns, whatever the path
-    struct Reopen {
+    FinGate fin{c, s};
+    // the histories are off again when this call returns
+    struct HistOff {
         mspms_ctx* c;
         hipStream_t s;
-        bool armed, hist_on;
-        ~Reopen() {
-            if (armed) (void)hipMemsetD32Async((hipDeviceptr_t)c->d_fin_on.p, 1, 1, s);
-            if (hist_on) {
-                LaunchCtx L = launch_ctx(c, s);
-                launch_set_hist(L, c->d_hist.p, HistDev{}, c->d_hstep.p);
-            }
+        bool on;
+        ~HistOff() {
+            if (!on) return;
+            LaunchCtx L = launch_ctx(c, s);
+            launch_set_hist(L, c->d_hist.p, HistDev{}, c->d_hstep.p);
         }
-    } reopen{c, s, false, false};
-    if (gate) {
-        HIPC(hipMemsetD32Async((hipDeviceptr_t)c->d_fin_on.p, 0, 1, s));
-        reopen.armed = true;
-    }
+    } hist_off{c, s, false};
+    if (gate) HIPC(fin.set(false));
     // the overflow snapshot counts this run's steps
     HIPC(hipMemsetAsync(c->d_snap_count.p, 0, sizeof(int), s));
     HistDev hd{};
@@ -1919,7 +1945,7 @@ extern "C" int mspms_vver_run_device(mspms_ctx* c, double* pos, double* vel, dou
                      c->fin.nb, c->d_hstep.p, c->any_vacuum ? c->d_huvac.p : nullptr};
         launch_set_hist(L, c->d_hist.p, hd, c->d_hstep.p);
         HIPC(hipGetLastError());
-        reopen.hist_on = true;
+        hist_off.on = true;
     }
     for (int t = 0; t < nsteps;) {
         // a graph of `per` steps while that many remain, then single steps
@@ -1928,8 +1954,7 @@ extern "C" int mspms_vver_run_device(mspms_ctx* c, double* pos, double* vel, dou
         if (gate && t + adv >= nsteps) {
             // the launch that holds the last step reduces its terms (the
             // other steps of a graph reduce theirs too: the last one wins)
-            HIPC(hipMemsetD32Async((hipDeviceptr_t)c->d_fin_on.p, 1, 1, s));
-            reopen.armed = false;
+            HIPC(fin.set(true));
         }
         t += adv;
         if (grp) {
@@ -1997,8 +2022,12 @@ int enqueue_hmc_move(mspms_ctx* c, double* pos, double* vel, double* fl, double*
         ~Unset() { c->cur_rep_delt = nullptr; }
     } unset{c};
     c->cur_rep_delt = rep_delt;
+    // the acceptance test reads the last step's terms only: without the
+    // others' reduction (33 us of 290 us per step at 64 chains of 17,627
+    // molecules) the finalize launch clears the rebuild request alone
     for (int t = 0; t < nmd; t++)
-        if ((rc = enqueue_vver(c, pos, vel, fl, fs, delt, nstep_inner, lterms, sterms, ukin, s)))
+        if ((rc = enqueue_vver(c, pos, vel, fl, fs, delt, nstep_inner, lterms, sterms, ukin, s,
+                               t == nmd - 1)))
             return rc;
     launch_hmc_end(L, c->d_hmc.p, c->d_rng.p, lterms, sterms, ukin, pos, c->d_pos_old.p,
                    rep_delt);
@@ -2165,7 +2194,7 @@ int enqueue_nvt(mspms_ctx* c, double* pos, double* vel, double* fl, double* fs, 
     launch_nvt_outer(L, c->nvt_plan, P, nstep_inner, ukin);
     {
         ProfScope p(c, s, PROF_FINAL);
-        launch_finalize(c, L, lterms, sterms, nullptr);
+        launch_finalize(c, L, lterms, sterms, nullptr, c->d_fin_on.p);
     }
     HIPC(hipGetLastError());
     return 0;
@@ -2324,18 +2353,33 @@ extern "C" int mspms_nvt_run_device(mspms_ctx* c, double* pos, double* vel, doub
         return fail(MSPMS_EINVAL, "null argument");
     HIPC(hipSetDevice(c->device));
     hipStream_t s = stream ? (hipStream_t)stream : c->stream;
+    // graphs of several steps, and the terms of the last step only, as in
+    // the NVE run
+    const int per = run_graph_steps(nsteps);
     if (use_graph) {
-        mspms_ctx::GraphKey k{pos, vel, fl, fs, lterms, sterms, ukin, delt, nstep_inner};
+        mspms_ctx::GraphKey k{pos, vel, fl, fs, lterms, sterms, ukin, delt, nstep_inner, per};
         int rc = ensure_graph(c, s, GRAPH_NVT, k, [&](hipStream_t cs) {
-            return enqueue_nvt(c, pos, vel, fl, fs, delt, nstep_inner, lterms, sterms, ukin, cs);
+            for (int q = 0; q < per; q++) {
+                int rq = enqueue_nvt(c, pos, vel, fl, fs, delt, nstep_inner, lterms, sterms, ukin,
+                                     cs);
+                if (rq) return rq;
+            }
+            return 0;
         });
         if (rc) return rc;
-        for (int t = 0; t < nsteps; t++) HIPC(hipGraphLaunch(c->graph_exec, s));
-        return 0;
     }
-    for (int t = 0; t < nsteps; t++) {
-        int rc = enqueue_nvt(c, pos, vel, fl, fs, delt, nstep_inner, lterms, sterms, ukin, s);
-        if (rc) return rc;
+    FinGate fin{c, s};
+    if (nsteps > 1) HIPC(fin.set(false));
+    for (int t = 0; t < nsteps;) {
+        const bool grp = use_graph && nsteps - t >= per;
+        t += grp ? per : 1;
+        if (fin.closed && t >= nsteps) HIPC(fin.set(true));
+        if (grp) {
+            HIPC(hipGraphLaunch(c->graph_exec, s));
+        } else {
+            int rc = enqueue_nvt(c, pos, vel, fl, fs, delt, nstep_inner, lterms, sterms, ukin, s);
+            if (rc) return rc;
+        }
     }
     return 0;
 }

@@ -176,6 +176,7 @@ struct FinBufs {
     const int* on;             // null, or a device flag: 0 = this pass only
                                //   clears the rebuild request (a step whose
                                //   terms nobody reads)
+    bool off;                  // the flag is known to be 0 when launching
     const HistDev* hist;       // null, or the run's history descriptor
     int* hstep;                // [nrep] next history slot of each replica
 };

@@ -942,9 +942,10 @@ void launch_finalize_long(const LaunchCtx& c, const int* col_cl0, const double* 
                           int* lstate, const double* ep_short, void* sterms,
                           const double* kin, double* ukin, const FinBufs& fb,
                           const FinAtoms* atoms) {
-    const dim3 grid(c.nrep * fb.nb);
     FinAtoms A{};
     if (atoms) A = *atoms;
+    // a pass that is off and has no closing pass is left with the request
+    const dim3 grid(fb.off && !atoms ? 1 : c.nrep * fb.nb);
     if (ep_short)
         hipLaunchKernelGGL(k_finalize<true>, grid, dim3(FIN_T), 0, c.stream, c.reps, col_cl0,
                            ep_pair, ip_pair, have_pair, ep_intra, have_intra, uk, have_recip,

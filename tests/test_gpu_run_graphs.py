@@ -1,0 +1,48 @@
+"""NVE and NVT device runs whose step counts give graphs of one to four steps,
+steps left over, and terms reduced for the last step only: the same state and
+the same terms as one-step calls without graphs.  FP64, whose sums all have a
+fixed order, so the two differ by nothing."""
+import numpy as np
+import pytest
+
+from mspms2_amd import configs
+from mspms2_amd.engine import LONG_TERMS_BYTES, SHORT_TERMS_BYTES, Engine
+from tests.util import system_of
+
+pytestmark = pytest.mark.gpu
+
+NSTEPS = (1, 2, 3, 5, 6, 8, 9, 66)
+
+
+@pytest.mark.parametrize("kind", ["nve", "nvt"])
+def test_runs_equal_single_steps(kind):
+    import torch
+    s = system_of(configs.water_box(n_side=3, L=9.4, rc=4.5, kappa=0.6, kmax=4, ksqmax=16, seed=8))
+    v0 = np.random.default_rng(2).standard_normal((3, s.natom)) * np.sqrt(s.treq / s.masses())
+    dev = torch.device("cuda:0")
+    t = lambda a: torch.tensor(a, dtype=torch.float64, device=dev).contiguous()  # noqa: E731
+    eng = Engine.replicas([s], precision="fp64")
+    eng.set_list_skin(0.0)  # no list, and so no order of sums, from an earlier run
+    x0, fl0, fs0 = eng.packed_positions(), eng.frclong()[0], eng.frcshort()[0]
+
+    def run(parts, graph):
+        if kind == "nvt":
+            eng.nvt_set(4.0 * s.natom, 2.0 * s.natom, s.treq, 3 * s.natom - 3)
+        bufs = [t(x0), t(v0), t(fl0), t(fs0)]
+        lt = torch.zeros(LONG_TERMS_BYTES // 8, dtype=torch.float64, device=dev)
+        st = torch.zeros(SHORT_TERMS_BYTES // 8, dtype=torch.float64, device=dev)
+        uk = torch.zeros(1, dtype=torch.float64, device=dev)
+        torch.cuda.synchronize()
+        call = eng.nvt_run_device if kind == "nvt" else eng.vver_run_device
+        for n in parts:
+            call(*bufs, 0.25 * s.delt, 2, n, lt, st, uk, graph=graph)
+        eng.sync()
+        return [b.cpu() for b in (*bufs, lt, st, uk)]
+
+    for n in NSTEPS:
+        print(f"{kind} {n} steps", flush=True)
+        want = run([1] * n, False)
+        for graph in (True, False):
+            for g, w in zip(run([n], graph), want):
+                assert torch.equal(g.view(torch.int64), w.view(torch.int64))
+    eng.close()
