@@ -2402,8 +2402,10 @@ int enqueue_npt(mspms_ctx* c, double* pos, double* vel, double* fl, double* fs, 
     {
         ProfScope p(c, s, PROF_BONDED);
         launch_npt_op(L, st, false, vel, fl, fs, lterms, sterms, deltby2, deltsby2, dt_outer4,
-                      dt_outer8, nullptr);
-        for (int ll = 0; ll < nstep_inner; ll++) {
+                      dt_outer8, nullptr, c->d_rmass.p);
+        const bool whole = launch_npt_inner_loop(L, c->d_terms.p, c->d_reps.p, st, pos, vel, fs,
+                                                 delts, deltsby2, nstep_inner, c->d_ep_short.p);
+        for (int ll = 0; ll < nstep_inner && !whole; ll++) {
             launch_npt_inner(L, c->d_reps.p, st, ll == 0, pos, vel, fs, delts, deltsby2);
             launch_bonded(L, c->d_species.p, c->d_terms.p, pos, pos + n, pos + 2 * n, fs, fs + n,
                           fs + 2 * n, c->d_ep_short.p);
@@ -2422,7 +2424,7 @@ int enqueue_npt(mspms_ctx* c, double* pos, double* vel, double* fl, double* fs, 
         launch_finalize(c, L, lterms, sterms, nullptr);
     }
     launch_npt_op(L, st, true, vel, fl, fs, lterms, sterms, deltby2, deltsby2, dt_outer4,
-                  dt_outer8, ukin);
+                  dt_outer8, ukin, c->d_rmass.p);
     HIPC(hipGetLastError());
     return 0;
 }

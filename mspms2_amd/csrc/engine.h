@@ -311,9 +311,15 @@ struct NptDev {
 };
 void launch_npt_op(const LaunchCtx& c, NptDev* st, bool end, double* vel, const double* fl,
                    const double* fs, const void* lterms, const void* sterms, double deltby2,
-                   double deltsby2, double dt_outer4, double dt_outer8, double* ukin);
+                   double deltsby2, double dt_outer4, double dt_outer8, double* ukin,
+                   const double* rmass);
 void launch_npt_inner(const LaunchCtx& c, RepDev* reps, NptDev* st, bool first, double* pos,
                       double* vel, const double* fs, double delts, double deltsby2);
+// the whole inner loop in one launch; false (and nothing launched) where the
+// molecules are too large for it
+bool launch_npt_inner_loop(const LaunchCtx& c, const TermDev* terms, RepDev* reps, NptDev* st,
+                           double* pos, double* vel, double* fs, double delts, double deltsby2,
+                           int nstep_inner, double* epart);
 void launch_kvec(const LaunchCtx& c, const RecipBufs& rb, int nrow);
 
 // Nose-Hoover NVT (k_nvt.hip)

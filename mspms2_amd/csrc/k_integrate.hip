@@ -16,6 +16,7 @@
 #include "engine.h"
 #include "sf_eval.h"
 #include "inner_terms.h"
+#include "npt_box.h"
 #include "terms.h"
 #include "wave.h"
 
@@ -401,15 +402,34 @@ __global__ void __launch_bounds__(64) k_respa_inner_tpm(
 // other).  A site's force is the sum of the NW copies in wave (= term)
 // order, as k_respa_inner_tpm sums its lane copies.  Molecules of up to NW
 // sites and NW terms.
-template <int NW>
+//
+// NPT: the inner loop of npt_respa (src/nptnh.c:152-211): the outer half
+// kicks and the last closing one are k_npt_op's, a drift scales the position
+// before and after (NB.st: the barostat's velocity), and the workgroups
+// behind those of the molecules move the replicas' boxes.  It is bound by the
+// latency of nstep_inner dependent steps either way; in one launch of 12 us
+// it replaces a launch of k_npt_inner and one of k_bonded per inner step
+// (8 inner steps, 999 molecules: 131 us).
+struct NptInner {
+    NptDev* st;
+    RepDev* reps;
+    int nrep;
+};
+
+template <int NW, bool NPT>
 __global__ void __launch_bounds__(64 * NW) k_respa_inner_tw(
     int nmol, const MolDev* __restrict__ mols, const SpeciesDev* __restrict__ species,
     const TermDev* __restrict__ terms, const SiteDev* __restrict__ sites, double* x, double* y,
     double* z, double* vx, double* vy, double* vz, const double* __restrict__ fxl,
     const double* __restrict__ fyl, const double* __restrict__ fzl, double* fxs, double* fys,
     double* fzs, double deltby2, double delts, double deltsby2, int nstep_inner, double* epart,
-    Status* st, const double* __restrict__ rep_delt, SfInner W, SnapOut SN) {
+    Status* st, const double* __restrict__ rep_delt, SfInner W, SnapOut SN, NptInner NB) {
 #pragma clang fp contract(off)
+    if (NPT && blockIdx.x * 64 >= nmol) {
+        const int r = (blockIdx.x - (nmol + 63) / 64) * (64 * NW) + threadIdx.x;
+        if (r < NB.nrep) npt_box(NB.reps[r], NB.st[r], delts, nstep_inner);
+        return;
+    }
     __shared__ double lx[NW * 64], ly[NW * 64], lz[NW * 64];
     __shared__ double cfx[NW][NW * 64], cfy[NW][NW * 64], cfz[NW][NW * 64];
     __shared__ double le[NW][5][64];
@@ -428,6 +448,7 @@ __global__ void __launch_bounds__(64 * NW) k_respa_inner_tw(
         if (w < nbt) T = terms[M.bterm0 + w];  // this wave's term, for every substep
         rep_steps(rep_delt, M.rep, nstep_inner, deltby2, delts, deltsby2);
     }
+    const double AA = NPT && live ? exp(deltsby2 * NB.st[rep].vbs) : 1.0;  // src/nptnh.c:157
     const bool own = live && w < na;      // site w of molecule m
     const bool term = live && w < nbt;    // term w of molecule m
     const int sl = w * 64 + mi;
@@ -448,9 +469,14 @@ __global__ void __launch_bounds__(64 * NW) k_respa_inner_tw(
         lx[sl] = pxo;
         ly[sl] = pyo;
         lz[sl] = pzo;
-        vxo = vx[i] + (deltby2 * fxl[i] * r_mass);
-        vyo = vy[i] + (deltby2 * fyl[i] * r_mass);
-        vzo = vz[i] + (deltby2 * fzl[i] * r_mass);
+        vxo = vx[i];
+        vyo = vy[i];
+        vzo = vz[i];
+        if (!NPT) {
+            vxo = vxo + (deltby2 * fxl[i] * r_mass);
+            vyo = vyo + (deltby2 * fyl[i] * r_mass);
+            vzo = vzo + (deltby2 * fzl[i] * r_mass);
+        }
         fxo = fxs[i];
         fyo = fys[i];
         fzo = fzs[i];
@@ -475,9 +501,19 @@ __global__ void __launch_bounds__(64 * NW) k_respa_inner_tw(
             vxo += (deltsby2 * fxo * r_mass);
             vyo += (deltsby2 * fyo * r_mass);
             vzo += (deltsby2 * fzo * r_mass);
+            if (NPT) {
+                pxo = pxo * AA;
+                pyo = pyo * AA;
+                pzo = pzo * AA;
+            }
             pxo = pxo + delts * vxo;
             pyo = pyo + delts * vyo;
             pzo = pzo + delts * vzo;
+            if (NPT) {
+                pxo = pxo * AA;
+                pyo = pyo * AA;
+                pzo = pzo * AA;
+            }
             lx[sl] = pxo;
             ly[sl] = pyo;
             lz[sl] = pzo;
@@ -517,9 +553,11 @@ __global__ void __launch_bounds__(64 * NW) k_respa_inner_tw(
             if (W.on)
                 usf_last = sf_inner_site(W, sites[site0 + w], rep, pxo, pyo, pzo, fxo, fyo, fzo,
                                          st);
-            vxo += (deltsby2 * fxo * r_mass);
-            vyo += (deltsby2 * fyo * r_mass);
-            vzo += (deltsby2 * fzo * r_mass);
+            if (!NPT || ll + 1 < nstep_inner) {
+                vxo += (deltsby2 * fxo * r_mass);
+                vyo += (deltsby2 * fyo * r_mass);
+                vzo += (deltsby2 * fzo * r_mass);
+            }
         }
     }
     if (own) {
@@ -749,10 +787,10 @@ void launch_respa_inner(const LaunchCtx& c, const SpeciesDev* species, const Ter
                        fzl, fxs, fys, fzs, deltby2, delts, deltsby2, nstep_inner, epart,        \
                        c.status, c.rep_delt, W, SN)
 #define RESPA_TW(NW)                                                                         \
-    hipLaunchKernelGGL(k_respa_inner_tw<NW>, dim3((c.nmol + 63) / 64), dim3(64 * NW), 0,          \
+    hipLaunchKernelGGL((k_respa_inner_tw<NW, false>), dim3((c.nmol + 63) / 64), dim3(64 * NW), 0, \
                        c.stream, c.nmol, c.mols, species, terms, c.sites, x, y, z, vx, vy, vz,    \
                        fxl, fyl, fzl, fxs, fys, fzs, deltby2, delts, deltsby2, nstep_inner,       \
-                       epart, c.status, c.rep_delt, W, SN)
+                       epart, c.status, c.rep_delt, W, SN, NptInner{})
 #define RESPA_TPM(NA, TPM)                                                                   \
     hipLaunchKernelGGL((k_respa_inner_tpm<NA, TPM>), dim3((c.nmol + 64 / TPM - 1) / (64 / TPM)), \
                        dim3(64), 0, c.stream, c.nmol, c.mols, species, terms, c.sites, x, y, z,  \
@@ -786,6 +824,26 @@ void launch_respa_inner(const LaunchCtx& c, const SpeciesDev* species, const Ter
 #undef RESPA_LDS
 #undef RESPA_TW
 #undef RESPA_TPM
+}
+
+bool launch_npt_inner_loop(const LaunchCtx& c, const TermDev* terms, RepDev* reps, NptDev* st,
+                           double* pos, double* vel, double* fs, double delts, double deltsby2,
+                           int nstep_inner, double* epart) {
+    const size_t n = (size_t)c.natom;
+    auto run = [&](auto kernel, int nw) {
+        const int boxes = (c.nrep + 64 * nw - 1) / (64 * nw);
+        hipLaunchKernelGGL(kernel, dim3((c.nmol + 63) / 64 + boxes), dim3(64 * nw), 0, c.stream,
+                           c.nmol, c.mols, nullptr, terms, c.sites, pos, pos + n, pos + 2 * n,
+                           vel, vel + n, vel + 2 * n, nullptr, nullptr, nullptr, fs, fs + n,
+                           fs + 2 * n, 0.0, delts, deltsby2, nstep_inner, epart, c.status,
+                           nullptr, SfInner{}, SnapOut{}, NptInner{st, reps, c.nrep});
+        return true;
+    };
+    const int most = std::max(c.max_mol_atoms, c.max_mol_terms);
+    if (most <= 1) return run(k_respa_inner_tw<1, true>, 1);
+    if (most <= 3) return run(k_respa_inner_tw<3, true>, 3);
+    if (most <= 4) return run(k_respa_inner_tw<4, true>, 4);
+    return false;
 }
 
 void launch_respa_final(const LaunchCtx& c, double* vx, double* vy, double* vz,

@@ -1,30 +1,32 @@
 // k_npt.hip -- NPT RESPA step on gfx950: npt_respa with the Nose-Hoover
 // thermostat / barostat operator npt_nh_operator (src/nptnh.c:10-234).
 //
-// Every phase that couples the atoms of a replica (sums of m v^2, scaling of
-// all positions, the box) runs as one workgroup per replica, with the
-// fixed-order workgroup sums of the NVT kernels; the box changes after every
-// inner step, so this kernel also rewrites the replica's box-dependent
-// tables that the force kernels read (RepDev: L, 1/L, cell sizes, and for
-// Ewald 2 pi / L, 2 pi / V, 2 pi / 3V) as the reference rewrites its
-// globals (src/nptnh.c:180-199), and k_kvec refreshes the Ewald weights
+// The sums of m v^2 run as one workgroup per replica, in a fixed order.  The
+// box changes with every inner step; the replica's box-dependent tables that
+// the force kernels read (RepDev: L, 1/L, cell sizes, and for Ewald 2 pi / L,
+// 2 pi / V, 2 pi / 3V) are rewritten as the reference rewrites its globals
+// (src/nptnh.c:180-199), and k_kvec refreshes the Ewald weights
 // exp(-B k^2) / k^2 of the new box before frclong.
 //   k_npt_op<START>   operator (src/nptnh.c:10-130); outer half kick
-//   k_npt_inner<FIRST> [previous inner step's closing half kick]; half kick,
-//                     x := AA (AA x + delts v), box *= exp(delts vbs)
-//   k_bonded          frcshort
-//   ... nstep_inner times, then k_kvec, frclong and the finalize pass, then
+//   inner loop: [previous inner step's closing half kick]; half kick,
+//               x := AA (AA x + delts v), box *= exp(delts vbs); frcshort.
+//               The barostat's velocity vbs stays as it is over the loop, so
+//               a molecule needs no other one: where molecules are small
+//               k_integrate.hip runs all of it in one launch
+//               (launch_npt_inner_loop), for larger ones each inner step is
+//               k_npt_inner<FIRST> and k_bonded
+//   then k_kvec, frclong and the finalize pass, then
 //   k_npt_op<END>     last inner closing kick, outer half kick, operator
 // FP64 in the reference's expression order; only the sums over atoms are
 // taken in a tree order.
 #include "engine.h"
+#include "npt_box.h"
 #include "wave.h"
 #include "../../include/mspms_gpu.h"
 
 namespace {
 
 constexpr int NPT_T = 1024;
-constexpr double NPT_PI = 3.141592653589793;  // src/defs.h:98
 
 __device__ double wg_sum_npt(double v, double* sh) {
     double a[1] = {v};
@@ -87,59 +89,102 @@ __device__ double npt_operator(NptDev& S, double mvsq, double vir_inter, double 
     return AA;
 }
 
+// Atoms of a replica whose velocities a thread keeps in registers between the
+// sum and the scaling (the others are read again).
+constexpr int NPT_KEEP = 4;
+
+// One workgroup per replica.  What bounds it is one chain of dependent steps
+// (loads, sum, the operator's exponentials and quotients, stores), so every
+// load of the chain's start is issued together, the reciprocal masses come
+// from the context's table, and one wave computes the operator while the
+// others wait for the scale (2,997 sites: start and end 12.8 and 14.0 us
+// before, 6.3 and 8.1 after).
 template <bool END>
 __global__ void __launch_bounds__(NPT_T) k_npt_op(
-    const RepDev* __restrict__ reps, const SiteDev* __restrict__ sites,
-    const int* __restrict__ atom_site, NptDev* __restrict__ st, double* __restrict__ vx,
-    double* __restrict__ vy, double* __restrict__ vz, const double* __restrict__ fxl,
-    const double* __restrict__ fyl, const double* __restrict__ fzl,
-    const double* __restrict__ fxs, const double* __restrict__ fys,
-    const double* __restrict__ fzs, const mspms_long_terms* __restrict__ lterms,
-    const mspms_short_terms* __restrict__ sterms, double deltby2, double deltsby2,
-    double dt_outer4, double dt_outer8, double* __restrict__ ukin) {
+    const RepDev* __restrict__ reps, const double* __restrict__ rmass, NptDev* __restrict__ st,
+    double* __restrict__ vx, double* __restrict__ vy, double* __restrict__ vz,
+    const double* __restrict__ fxl, const double* __restrict__ fyl,
+    const double* __restrict__ fzl, const double* __restrict__ fxs,
+    const double* __restrict__ fys, const double* __restrict__ fzs,
+    const mspms_long_terms* __restrict__ lterms, const mspms_short_terms* __restrict__ sterms,
+    double deltby2, double deltsby2, double dt_outer4, double dt_outer8,
+    double* __restrict__ ukin) {
 #pragma clang fp contract(off)
     __shared__ double sh[16];
+    __shared__ double scale;
     const int r = blockIdx.x;
-    const RepDev& R = reps[r];
-    NptDev S = st[r];
-    const int a0 = R.atom0, a1 = R.atom0 + R.natom;
+    const int a0 = reps[r].atom0, natom = reps[r].natom, a1 = a0 + natom;
+    const double vir_inter = lterms[r].virial_inter, vir_intra = sterms[r].virial_intra;
     double m2 = 0.0;
-    for (int i = a0 + threadIdx.x; i < a1; i += NPT_T) {
-        const double r_mass = rmass(sites, atom_site, i);
-        double a = vx[i], b = vy[i], c = vz[i];
+    double va[NPT_KEEP], vb[NPT_KEEP], vc[NPT_KEEP], rm[NPT_KEEP];
+    double la[NPT_KEEP], lb[NPT_KEEP], lc[NPT_KEEP];
+    // closing half kick of the last inner step (src/nptnh.c:201-210) and the
+    // outer one with the new long forces (:214-223), then m v^2
+    auto first = [&](int i, double& a, double& b, double& c, double& r_mass, double& fa,
+                     double& fb, double& fc) {
+        a = vx[i];
+        b = vy[i];
+        c = vz[i];
+        r_mass = rmass[i];
+        fa = fxl[i];
+        fb = fyl[i];
+        fc = fzl[i];
         if (END) {
-            // closing half kick of the last inner step (src/nptnh.c:201-210)
-            // and the outer one with the new long forces (:214-223)
             a += (deltsby2 * fxs[i] * r_mass);
             b += (deltsby2 * fys[i] * r_mass);
             c += (deltsby2 * fzs[i] * r_mass);
-            a += (deltby2 * fxl[i] * r_mass);
-            b += (deltby2 * fyl[i] * r_mass);
-            c += (deltby2 * fzl[i] * r_mass);
-            vx[i] = a;
-            vy[i] = b;
-            vz[i] = c;
+            a += (deltby2 * fa * r_mass);
+            b += (deltby2 * fb * r_mass);
+            c += (deltby2 * fc * r_mass);
         }
-        m2 += (a * a + b * b + c * c) / r_mass;
-    }
-    const double mvsq = wg_sum_npt(m2, sh);
-    const double AA = npt_operator(S, mvsq, lterms[r].virial_inter, sterms[r].virial_intra,
-                                   R.natom, deltby2, deltby2, dt_outer4, dt_outer8,
-                                   threadIdx.x == 0, END && ukin ? ukin + r : nullptr);
-    for (int i = a0 + threadIdx.x; i < a1; i += NPT_T) {
-        double a = vx[i] * AA, b = vy[i] * AA, c = vz[i] * AA;
+        return (a * a + b * b + c * c) / r_mass;
+    };
+    // the scale, and at the start the outer half kick (src/nptnh.c:141-150)
+    auto second = [&](int i, double AA, double a, double b, double c, double r_mass, double fa,
+                      double fb, double fc) {
+        a = a * AA;
+        b = b * AA;
+        c = c * AA;
         if (!END) {
-            // outer half kick (src/nptnh.c:141-150)
-            const double r_mass = rmass(sites, atom_site, i);
-            a += (deltby2 * fxl[i] * r_mass);
-            b += (deltby2 * fyl[i] * r_mass);
-            c += (deltby2 * fzl[i] * r_mass);
+            a += (deltby2 * fa * r_mass);
+            b += (deltby2 * fb * r_mass);
+            c += (deltby2 * fc * r_mass);
         }
         vx[i] = a;
         vy[i] = b;
         vz[i] = c;
+    };
+    const int i0 = a0 + threadIdx.x;
+#pragma unroll
+    for (int k = 0; k < NPT_KEEP; k++) {
+        const int i = i0 + k * NPT_T;
+        if (i < a1) m2 += first(i, va[k], vb[k], vc[k], rm[k], la[k], lb[k], lc[k]);
     }
-    if (threadIdx.x == 0) st[r] = S;
+    for (int i = i0 + NPT_KEEP * NPT_T; i < a1; i += NPT_T) {
+        double a, b, c, q, fa, fb, fc;
+        m2 += first(i, a, b, c, q, fa, fb, fc);
+        if (END) {
+            vx[i] = a;
+            vy[i] = b;
+            vz[i] = c;
+        }
+    }
+    const double mvsq = wg_sum_npt(m2, sh);
+    if (threadIdx.x < 64) {
+        const double AA = npt_operator(st[r], mvsq, vir_inter, vir_intra, natom, deltby2, deltby2,
+                                       dt_outer4, dt_outer8, threadIdx.x == 0,
+                                       END && ukin ? ukin + r : nullptr);
+        if (threadIdx.x == 0) scale = AA;
+    }
+    __syncthreads();
+    const double AA = scale;
+#pragma unroll
+    for (int k = 0; k < NPT_KEEP; k++) {
+        const int i = i0 + k * NPT_T;
+        if (i < a1) second(i, AA, va[k], vb[k], vc[k], rm[k], la[k], lb[k], lc[k]);
+    }
+    for (int i = i0 + NPT_KEEP * NPT_T; i < a1; i += NPT_T)
+        second(i, AA, vx[i], vy[i], vz[i], rmass[i], fxl[i], fyl[i], fzl[i]);
 }
 
 template <bool FIRST>
@@ -183,25 +228,7 @@ __global__ void __launch_bounds__(NPT_T) k_npt_inner(
     // every atom of the replica has read the old box before it changes
     __syncthreads();
     if (threadIdx.x != 0) return;
-    // src/nptnh.c:179-199
-    const double expfactor = exp(delts * vbs);
-    const int nc[3] = {R.ncx, R.ncy, R.ncz};
-    for (int d = 0; d < 3; d++) {
-        R.L[d] = R.L[d] * expfactor;
-        R.invL[d] = 1.0 / R.L[d];
-        R.h[d] = R.L[d] / nc[d];
-        R.inv_h[d] = 1.0 / R.h[d];
-    }
-    const double boxv = R.L[0] * R.L[1] * R.L[2];
-    S->boxv = boxv;
-    double p = 0.0;
-    for (int k = 0; k < S->nlrc; k++) p += S->lrc[k] / boxv / boxv;
-    S->pljlrc = p;
-    if (R.charge_type == MSPMS_ELEC_EWALD) {
-        R.vfactor = 2.0 * NPT_PI / boxv;
-        for (int d = 0; d < 3; d++) R.twopi_l[d] = 2.0 * NPT_PI / R.L[d];
-        R.twopi_over_3v = 2.0 * NPT_PI / 3.0 / boxv;
-    }
+    npt_box(R, *S, delts, 1);
 }
 
 // Ewald weights exp(-B k^2) / k^2 of the current box, one thread per k row
@@ -228,18 +255,19 @@ __global__ void __launch_bounds__(256) k_kvec(int nrow, const KRow* __restrict__
 
 void launch_npt_op(const LaunchCtx& c, NptDev* st, bool end, double* vel, const double* fl,
                    const double* fs, const void* lterms, const void* sterms, double deltby2,
-                   double deltsby2, double dt_outer4, double dt_outer8, double* ukin) {
+                   double deltsby2, double dt_outer4, double dt_outer8, double* ukin,
+                   const double* rmass) {
     const size_t n = (size_t)c.natom;
     auto* lt = (const mspms_long_terms*)lterms;
     auto* sm = (const mspms_short_terms*)sterms;
     if (end)
         hipLaunchKernelGGL(k_npt_op<true>, dim3(c.nrep), dim3(NPT_T), 0, c.stream, c.reps,
-                           c.sites, c.atom_site, st, vel, vel + n, vel + 2 * n, fl, fl + n,
+                           rmass, st, vel, vel + n, vel + 2 * n, fl, fl + n,
                            fl + 2 * n, fs, fs + n, fs + 2 * n, lt, sm, deltby2, deltsby2,
                            dt_outer4, dt_outer8, ukin);
     else
         hipLaunchKernelGGL(k_npt_op<false>, dim3(c.nrep), dim3(NPT_T), 0, c.stream, c.reps,
-                           c.sites, c.atom_site, st, vel, vel + n, vel + 2 * n, fl, fl + n,
+                           rmass, st, vel, vel + n, vel + 2 * n, fl, fl + n,
                            fl + 2 * n, fs, fs + n, fs + 2 * n, lt, sm, deltby2, deltsby2,
                            dt_outer4, dt_outer8, ukin);
 }
