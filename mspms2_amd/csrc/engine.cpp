@@ -118,6 +118,7 @@ struct mspms_ctx {
     int charge_union = MSPMS_ELEC_NONE;  // charge type shared by the replicas
     bool any_intra = false, any_bonded = false, any_recip = false, any_sf = false;
     int max_mol_terms = 0;  // most bonded terms of one molecule (any species)
+    int max_mol_intra = 0;  // most intramolecular pair terms
     bool sf_split = false;  // the solid-fluid wall in frcshort / the inner loop
     bool any_vacuum = false, any_coul = false;
     int want_hash = -1;                  // -1: FP64 only
@@ -315,6 +316,7 @@ LaunchCtx launch_ctx(mspms_ctx* c, hipStream_t s) {
     L.max_mol_atoms = 0;
     for (const SpeciesHost& q : c->sp) L.max_mol_atoms = std::max(L.max_mol_atoms, q.natom);
     L.max_mol_terms = c->max_mol_terms;
+    L.max_mol_intra = c->max_mol_intra;
     L.rep_delt = c->cur_rep_delt;
     L.snap = nullptr;
     L.snap_count = nullptr;
@@ -668,7 +670,7 @@ int build(mspms_ctx* c) {
     std::vector<SpeciesDev> spd;
     std::vector<TermDev> terms;
     c->any_intra = c->any_bonded = false;
-    c->max_mol_terms = 0;
+    c->max_mol_terms = c->max_mol_intra = 0;
     for (int k = 0; k < ns; k++) {
         const SpeciesHost& q = c->sp[k];
         SpeciesDev d{};
@@ -756,6 +758,7 @@ int build(mspms_ctx* c) {
         }
         d.nbterm = (int)terms.size() - d.bterm0;
         c->max_mol_terms = std::max(c->max_mol_terms, d.nbterm);
+        c->max_mol_intra = std::max(c->max_mol_intra, d.nintra);
         if (d.nintra > 0) c->any_intra = true;
         if (d.nbterm > 0) c->any_bonded = true;
         spd.push_back(d);

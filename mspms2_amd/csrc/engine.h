@@ -202,6 +202,7 @@ struct LaunchCtx {
     int natom, nmol, nsite, nrep;
     int max_mol_atoms;        // largest molecule (atoms) of any species
     int max_mol_terms;        // most bonded terms of one molecule of any species
+    int max_mol_intra;        // most intramolecular pair terms, likewise
     int pair_wpc;             // waves per i-cluster of the mixed pair kernel
     const SiteDev* sites;
     const MolDev* mols;

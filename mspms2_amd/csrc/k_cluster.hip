@@ -716,7 +716,10 @@ void launch_cluster_build(const LaunchCtx& c, ClusterBufs& b, const double* x, c
     // the last binning workgroup scans the cells.  1024 threads scan, and
     // arrive, faster where there are many (8,813 cells: 24.7 against 34.3 us;
     // 6,144: 18.3 against 25.2); at 1,331 cells both take 13.0, and smaller
-    // systems would leave CUs idle while they bin.
+    // systems would leave CUs idle while they bin.  But a workgroup of 16 waves
+    // also waits for a CU free of the side stream's work on the steps that
+    // build nothing (98,304 sites: 125 us behind the structure factors), so
+    // they are for calls that always build.
     auto bin = [&](auto kernel, int nt) {
         hipLaunchKernelGGL(kernel, dim3((c.natom + nt - 1) / nt), dim3(nt), 0, c.stream, c.natom,
                            x, y, z, c.atom_site, c.atom_mol, c.sites, c.mols, c.reps, b.atom_cell,
@@ -724,7 +727,7 @@ void launch_cluster_build(const LaunchCtx& c, ClusterBufs& b, const double* x, c
                            c.status, b.lstate, b.ncell, b.ncol, b.cell_start, b.col_cell0,
                            b.col_cl0, b.cl_col, b.ncl_total, b.maxcl, b.bin_ctr);
     };
-    if (b.ncell > 2048)
+    if (b.ncell > 2048 && (force || half_skin2 == 0.0))
         bin(k_bin_scan<1024>, 1024);
     else
         bin(k_bin_scan<256>, 256);

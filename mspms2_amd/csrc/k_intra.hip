@@ -254,6 +254,127 @@ __global__ void __launch_bounds__(256) k_intra(int nmol, const MolDev* __restric
             kick_atom(K, base + k, fx, fy, fz);
 }
 
+// k_intra without the adjoint, one term per wave: a workgroup of NW waves takes
+// 64 molecules (lane = molecule), wave w computes term w and owns site w.  A
+// thread per molecule steps through its terms one after another, each a
+// chain of a square root, quotients, erfc and exp, on few waves; the chain is
+// what bounds this kernel, which runs ahead of the reciprocal kernels on their
+// stream (or of the step's last kernel where there are none).  A site's force is the sum of its terms' in term
+// order, as the energies are.  Molecules of up to NW sites and NW terms
+// (us, by a thread per molecule and by this kernel: water of 648 sites 12.8
+// and 4.5, of 12,288 13.5 and 4.4, of 98,304 20 and 6.5; butane, 70,508 sites,
+// 12.2 and 7.6).
+template <int NW>
+__global__ void __launch_bounds__(64 * NW) k_intra_tw(
+    int nmol, const MolDev* __restrict__ mols, const RepDev* __restrict__ reps,
+    const SiteDev* __restrict__ sites, const TermDev* __restrict__ terms,
+    const double* __restrict__ x, const double* __restrict__ y, const double* __restrict__ z,
+    double* fx, double* fy, double* fz, double* epart, Kick K, int zero_first) {
+    __shared__ double sf[3][NW][64];   // a term's force on its first site
+    __shared__ double le[4][NW][64];
+    __shared__ int pr[NW][64];         // a term's sites (0xff: none) and is_long
+    const int w = threadIdx.x >> 6, mi = threadIdx.x & 63;
+    const int m = blockIdx.x * 64 + mi;
+    const bool live = m < nmol;
+    MolDev M{};
+    if (live) M = mols[m];
+    const bool term = live && w < M.nintra;
+    const int base = M.atom0;
+    TermDev T{};
+    SiteDev a{}, b{};
+    double rx = 0.0, ry = 0.0, rz = 0.0;
+    bool lng = false;
+    const RepDev& R = reps[M.rep];
+    if (term) {
+#pragma clang fp contract(off)
+        T = terms[M.term0 + w];
+        a = sites[M.site0 + T.idx[0]];
+        b = sites[M.site0 + T.idx[1]];
+        const int ii = base + T.idx[0], jj = base + T.idx[1];
+        rx = x[ii] - x[jj];
+        ry = y[ii] - y[jj];
+        rz = z[ii] - z[jj];
+        lng = is_long(R, rx, ry, rz);
+    }
+    pr[w][mi] = term ? T.idx[0] | T.idx[1] << 8 | (int)lng << 16 | (T.kind == TERM_PAIR14) << 17
+                     : 0xffff;
+    __syncthreads();
+    IntraAcc acc = {0.0, 0.0, 0.0, 0.0};
+    // entry 0: the first site's force (entry 1, the second's, is its negative)
+    double gx[2] = {0.0, 0.0}, gy[2] = {0.0, 0.0}, gz[2] = {0.0, 0.0};
+    const GradOut none{nullptr, nullptr, nullptr};
+    const bool ghost = a.ghost == MSPMS_GHOST_FULL || b.ghost == MSPMS_GHOST_FULL;
+    if (term && !(lng && ghost)) {
+        const bool p14 = T.kind == TERM_PAIR14;
+        // 1-4 pairs go by what the last 1-2 / 1-3 term before them left
+        // (src/frclong.c:622, :632 compare, not assign)
+        bool same = true;
+        if (p14)
+            for (int c = 0; c < w; c++)
+                if (!(pr[c][mi] >> 17 & 1)) same = !(pr[c][mi] >> 16 & 1);
+        const bool image = p14 ? !same : lng;
+        if (image || p14) {
+            double mx = rx, my = ry, mz = rz;
+            if (image) {
+                mx = mic(rx, R.L[0]);
+                my = mic(ry, R.L[1]);
+                mz = mic(rz, R.L[2]);
+                // restored through int variables (src/frclong.c:223): truncation
+                rx = (double)(int)rx;
+                ry = (double)(int)ry;
+                rz = (double)(int)rz;
+            }
+            if (!image || (a.ghost != MSPMS_GHOST_LJ && b.ghost != MSPMS_GHOST_LJ))
+                intra_lj<false>(R, a, b, 0, 1, mx, my, mz, image ? 1.0 : R.f0, acc, gx, gy, gz,
+                                none);
+        }
+        intra_elec<false>(R, a.charge * b.charge, a.charge, b.charge, 0, 1, rx, ry, rz, !p14, acc,
+                          gx, gy, gz, none);
+    }
+    sf[0][w][mi] = gx[0];
+    sf[1][w][mi] = gy[0];
+    sf[2][w][mi] = gz[0];
+    le[0][w][mi] = acc.uvdw;
+    le[1][w][mi] = acc.ureal;
+    le[2][w][mi] = acc.uexcl;
+    le[3][w][mi] = acc.vir;
+    __syncthreads();
+    if (live && w < M.natom) {
+        const int i = base + w;
+        double ax = zero_first ? 0.0 : fx[i], ay = zero_first ? 0.0 : fy[i],
+               az = zero_first ? 0.0 : fz[i];
+#pragma unroll
+        for (int c = 0; c < NW; c++) {
+            const int p = pr[c][mi];
+            if ((p & 0xff) == w) {
+                ax += sf[0][c][mi];
+                ay += sf[1][c][mi];
+                az += sf[2][c][mi];
+            }
+            if ((p >> 8 & 0xff) == w) {
+                ax -= sf[0][c][mi];
+                ay -= sf[1][c][mi];
+                az -= sf[2][c][mi];
+            }
+        }
+        fx[i] = ax;
+        fy[i] = ay;
+        fz[i] = az;
+        // the molecule's long forces are final
+        if (K.vx) kick_atom(K, i, fx, fy, fz);
+    }
+    if (live && w == 0) {
+        double* ep = epart + (size_t)m * 4;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            double e = 0.0;
+#pragma unroll
+            for (int c = 0; c < NW; c++) e += le[k][c][mi];
+            ep[k] = e;
+        }
+    }
+}
+
 __global__ void __launch_bounds__(256) k_bonded(int nmol, const MolDev* __restrict__ mols,
                                                 const SpeciesDev* __restrict__ species,
                                                 const TermDev* __restrict__ terms,
@@ -861,7 +982,19 @@ void launch_intra(const LaunchCtx& c, const SpeciesDev* species, const TermDev* 
                   const double* frec, const Kick* kick, bool zero_first) {
     int g = (c.nmol + 255) / 256;
     const Kick K = kick ? *kick : Kick{};
-    if (gq)
+    auto by_term = [&](auto kernel, int nw) {
+        hipLaunchKernelGGL(kernel, dim3((c.nmol + 63) / 64), dim3(64 * nw), 0, c.stream, c.nmol,
+                           c.mols, c.reps, c.sites, terms, x, y, z, fx, fy, fz, epart, K,
+                           zero_first ? 1 : 0);
+    };
+    const int most = std::max(c.max_mol_atoms, c.max_mol_intra);
+    if (!gq && !frec && most <= 3)
+        by_term(k_intra_tw<3>, 3);
+    else if (!gq && !frec && most <= 4)
+        by_term(k_intra_tw<4>, 4);
+    else if (!gq && !frec && most <= 6)
+        by_term(k_intra_tw<6>, 6);
+    else if (gq)
         hipLaunchKernelGGL(k_intra<true>, dim3(g), dim3(256), 0, c.stream, c.nmol, c.mols, c.reps,
                            c.sites, species, terms, x, y, z, fx, fy, fz, epart,
                            GradOut{gq, ge, gs}, c.natom, frec, K, zero_first ? 1 : 0);
