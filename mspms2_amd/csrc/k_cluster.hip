@@ -21,6 +21,7 @@
 //   k_plist    one wave per i-cluster: j-clusters whose boxes come within
 //              rc_list, compacted with a wave ballot (deterministic order)
 // The ranks make the final order independent of atomic arrival order.
+// Up to 1,024 atoms k_build_small does all but the last in one workgroup.
 //
 // Reuse: a list built with rc_list = cutoff + skin holds every pair within
 // the cutoff while no atom has moved more than skin/2 since the build (the
@@ -37,26 +38,24 @@
 
 namespace {
 
-__global__ void __launch_bounds__(64) k_list_check(
-    int natom, int nslot, const double* __restrict__ x, const double* __restrict__ y,
-    const double* __restrict__ z, const int* __restrict__ atom_site,
+// One atom and one slot (index t of both; adjacent lanes take adjacent ones):
+// does the atom's displacement ask for a new list?  ls_valid, ls_layout: the
+// list's state.
+__device__ inline bool check_one(
+    int t, int ls_valid, int ls_layout, int natom, int nslot, const double* __restrict__ x,
+    const double* __restrict__ y, const double* __restrict__ z, const int* __restrict__ atom_site,
     const SiteDev* __restrict__ sites, double* __restrict__ fx, double* __restrict__ fy,
     double* __restrict__ fz, const double4* __restrict__ atom_x0,
     const int* __restrict__ ncl_total, int maxcl, const int* __restrict__ slot_orig,
     const double4* __restrict__ slot_w64, const double4* __restrict__ cl_center,
     double4* __restrict__ slot_x64, float4* __restrict__ slot_off, float4* __restrict__ cl_box,
-    double* __restrict__ fslot, int* lstate, double half_skin2, int force, int half,
-    const HistDev* hist) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    // a device run recording histories: this call begins the next step
-    if (t == 0 && hist && hist->on) *hist->tick += 1;
+    double* __restrict__ fslot, double half_skin2, int force, int half) {
     // The kernel is a short chain of dependent loads on a few waves per CU:
     // every load that depends on no other (list state, this thread's atom
     // and slot) is issued before any is used, and only the slot's atom
     // position waits for the slot's atom index.  Slot data read here before
     // the first build are never used (the list is not valid then).
     const bool in_atom = t < natom, in_slot = t < nslot;
-    const int ls_valid = lstate[LS_VALID], ls_layout = lstate[LS_LAYOUT];
     const int ncl = min(*ncl_total, maxcl);
     const int site = in_atom ? atom_site[t] : 0;
     const double4 p0t = in_atom ? atom_x0[t] : make_double4(0.0, 0.0, 0.0, 0.0);
@@ -136,6 +135,26 @@ __global__ void __launch_bounds__(64) k_list_check(
             cl_box[2 * c + 1] = make_float4(0.f, 0.f, 0.f, 0.f);
         }
     }
+    return need;
+}
+
+__global__ void __launch_bounds__(64) k_list_check(
+    int natom, int nslot, const double* __restrict__ x, const double* __restrict__ y,
+    const double* __restrict__ z, const int* __restrict__ atom_site,
+    const SiteDev* __restrict__ sites, double* __restrict__ fx, double* __restrict__ fy,
+    double* __restrict__ fz, const double4* __restrict__ atom_x0,
+    const int* __restrict__ ncl_total, int maxcl, const int* __restrict__ slot_orig,
+    const double4* __restrict__ slot_w64, const double4* __restrict__ cl_center,
+    double4* __restrict__ slot_x64, float4* __restrict__ slot_off, float4* __restrict__ cl_box,
+    double* __restrict__ fslot, int* lstate, double half_skin2, int force, int half,
+    const HistDev* hist) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    // a device run recording histories: this call begins the next step
+    if (t == 0 && hist && hist->on) *hist->tick += 1;
+    const bool need =
+        check_one(t, lstate[LS_VALID], lstate[LS_LAYOUT], natom, nslot, x, y, z, atom_site, sites,
+                  fx, fy, fz, atom_x0, ncl_total, maxcl, slot_orig, slot_w64, cl_center, slot_x64,
+                  slot_off, cl_box, fslot, half_skin2, force, half);
     // one atomic per wave, and none once the request is seen set: atomics
     // on one address from every wave of a large system serialize
     if (__ballot(need) && (threadIdx.x & 63) == 0 &&
@@ -218,6 +237,8 @@ __device__ int block_exscan(int v, int* sh, int& total) {
     __syncthreads();
     return ex;
 }
+
+constexpr int SMALL_T = 1024;  // k_build_small's workgroup
 
 // Cells per pass of scan_cells: NT * SCAN_PER<NT> counts staged in LDS.
 template <int NT>
@@ -488,6 +509,71 @@ __global__ void __launch_bounds__(1024) k_place_bbox(
                   slot_info, slot_w64, slot_off, slot_par, cl_center, cl_ext, cl_box);
 }
 
+// k_list_check, k_bin_scan, k_scatter and k_place_bbox of a small system by one
+// workgroup, with barriers in place of the launches: where the list is
+// reused, as on most steps of a run, the three launches after the check do
+// nothing, at about 2 us each in a graph.  Buffers that one phase writes and a later
+// one reads carry no __restrict__ here.
+__global__ void __launch_bounds__(SMALL_T) k_build_small(
+    int natom, int nslot, const double* __restrict__ x, const double* __restrict__ y,
+    const double* __restrict__ z, const int* __restrict__ atom_site,
+    const int* __restrict__ atom_mol, const SiteDev* __restrict__ sites,
+    const MolDev* __restrict__ mols, const RepDev* __restrict__ reps, double* fx, double* fy,
+    double* fz, double4* atom_x0, int* ncl_total, int maxcl, int* slot_orig, int2* slot_info,
+    double4* slot_w64, double4* slot_x64, float4* slot_off, float4* slot_par, double4* cl_center,
+    float4* cl_ext, float4* cl_box, double* fslot, int* atom_cell, int* atom_slot,
+    double* atom_wz, int* cell_count, int* cell_start, int* cell_members,
+    const int* __restrict__ col_cell0, int* col_cl0, int* cl_col,
+    const int* __restrict__ col_rep, int* atom_gslot, int ncell, int ncol, Status* st,
+    int* lstate, double half_skin2, int force, int half, const HistDev* hist) {
+    __shared__ int sh[32];
+    __shared__ int stage[SCAN_LDS<SMALL_T>];
+    const int tid = threadIdx.x;
+    if (tid == 0 && hist && hist->on) *hist->tick += 1;
+    const int ls_valid = lstate[LS_VALID], ls_layout = lstate[LS_LAYOUT];
+    bool need = false;
+    for (int t0 = 0; t0 < max(natom, nslot); t0 += SMALL_T)
+        need |= check_one(t0 + tid, ls_valid, ls_layout, natom, nslot, x, y, z, atom_site, sites,
+                          fx, fy, fz, atom_x0, ncl_total, maxcl, slot_orig, slot_w64, cl_center,
+                          slot_x64, slot_off, cl_box, fslot, half_skin2, force, half);
+    // a request that is already there (a list reset) stands
+    if (!__syncthreads_or(need || lstate[LS_NEED])) return;
+    for (int i = tid; i < natom; i += SMALL_T)
+        bin_atom(i, x, y, z, atom_site, atom_mol, sites, mols, reps, atom_cell, atom_slot, atom_wz,
+                 cell_count, fx, fy, fz, atom_gslot, st);
+    __syncthreads();
+    scan_cells<SMALL_T>(ncell, ncol, cell_count, cell_start, col_cell0, col_cl0, cl_col, ncl_total,
+                        maxcl, st, sh, stage);
+    __syncthreads();
+    for (int i = tid; i < natom; i += SMALL_T) {
+        const int c = atom_cell[i];
+        if (c >= 0) cell_members[cell_start[c] + atom_slot[i]] = i;
+    }
+    __syncthreads();
+    // a wave per column
+    const int lane = tid & 63, w = tid >> 6, nw = SMALL_T / 64;
+    for (int col = w; col < ncol; col += nw) {
+        const int m0 = cell_start[col_cell0[col]], m1 = cell_start[col_cell0[col + 1]];
+        for (int m = m0 + lane; m < m1; m += 64)
+            place_atom(cell_members[m], col, m0, x, y, z, atom_cell, atom_wz, cell_start,
+                       cell_members, atom_mol, atom_site, mols, reps, col_cl0, slot_orig,
+                       slot_info, slot_x64, slot_w64, atom_x0, atom_gslot, sites, maxcl);
+    }
+    __syncthreads();
+    for (int col = w; col < ncol; col += nw) {
+        const int m0 = cell_start[col_cell0[col]], m1 = cell_start[col_cell0[col + 1]];
+        const int cl0 = col_cl0[col], c_end = min(col_cl0[col + 1], maxcl);
+        for (int t0 = MSPMS_CL * cl0; t0 < MSPMS_CL * c_end; t0 += 64)
+            bbox_slot(t0 + lane, c_end, col, m1 - m0, cl0, col_rep, sites, slot_orig, slot_info,
+                      slot_w64, slot_off, slot_par, cl_center, cl_ext, cl_box);
+    }
+    if (tid == 0) {
+        lstate[LS_NEED] = 1;
+        lstate[LS_VALID] = *ncl_total <= maxcl;
+        lstate[LS_BUILDS] += 1;
+    }
+}
+
 // One wave per i-cluster.  Candidate columns cover the x/y range of the
 // i-box widened by rc_list (periodic, each wrapped column at most once).
 // A column's clusters are in wrapped-z order (cells by cz, atoms in a cell
@@ -706,46 +792,61 @@ void launch_cluster_build(const LaunchCtx& c, ClusterBufs& b, const double* x, c
     const int T = 256;
     int gA = (c.natom + T - 1) / T;
     const int nslot = b.maxcl * MSPMS_CL;
-    // one-wave workgroups: the check is a short chain of dependent loads,
-    // which more, smaller workgroups spread over more CUs (0.9 us per step)
-    hipLaunchKernelGGL(k_list_check, dim3((std::max(c.natom, nslot) + 63) / 64), dim3(64), 0,
-                       c.stream, c.natom, nslot, x, y, z, c.atom_site, c.sites, fx, fy, fz,
-                       b.atom_x0, b.ncl_total, b.maxcl, b.slot_orig, b.slot_w64, b.cl_center,
-                       b.slot_x64, b.slot_off, b.cl_box, b.fslot, b.lstate, half_skin2, force,
-                       b.half, b.hist);
-    // the last binning workgroup scans the cells.  1024 threads scan, and
-    // arrive, faster where there are many (8,813 cells: 24.7 against 34.3 us;
-    // 6,144: 18.3 against 25.2); at 1,331 cells both take 13.0, and smaller
-    // systems would leave CUs idle while they bin.  But a workgroup of 16 waves
-    // also waits for a CU free of the side stream's work on the steps that
-    // build nothing (98,304 sites: 125 us behind the structure factors), so
-    // they are for calls that always build.
-    auto bin = [&](auto kernel, int nt) {
-        hipLaunchKernelGGL(kernel, dim3((c.natom + nt - 1) / nt), dim3(nt), 0, c.stream, c.natom,
-                           x, y, z, c.atom_site, c.atom_mol, c.sites, c.mols, c.reps, b.atom_cell,
-                           b.atom_slot, b.atom_wz, b.cell_count, fx, fy, fz, b.atom_gslot,
-                           c.status, b.lstate, b.ncell, b.ncol, b.cell_start, b.col_cell0,
-                           b.col_cl0, b.cl_col, b.ncl_total, b.maxcl, b.bin_ctr);
-    };
-    if (b.ncell > 2048 && (force || half_skin2 == 0.0))
-        bin(k_bin_scan<1024>, 1024);
-    else
-        bin(k_bin_scan<256>, 256);
-    hipLaunchKernelGGL(k_scatter, dim3(gA), dim3(T), 0, c.stream, c.natom, b.atom_cell,
-                       b.atom_slot, b.cell_start, b.cell_members, b.lstate);
-    // threads for 1.25 times the mean column, up to 1024 (a column of a long
-    // box holds thousands of atoms): a workgroup much larger than its column
-    // idles (70,508 atoms in 1,600 columns: 28.6 us with 1024 threads, 13.5
-    // with 64), and where no list is built it still waits for a CU with 16
-    // free waves.
-    int tp = 64;
-    while (tp < 1024 && (double)tp * b.ncol < 1.25 * c.natom) tp *= 2;
-    hipLaunchKernelGGL(k_place_bbox, dim3(b.ncol), dim3(tp), 0, c.stream, b.ncol, x, y, z,
-                       b.atom_cell, b.atom_wz, b.cell_start, b.cell_members, c.atom_mol,
-                       c.atom_site, c.mols, c.reps, b.col_cell0, b.col_cl0, b.col_rep,
-                       b.ncl_total, b.slot_orig, b.slot_info, b.slot_x64, b.slot_w64, b.atom_x0,
-                       b.atom_gslot, c.sites, b.slot_off, b.slot_par, b.cl_center, b.cl_ext,
-                       b.cl_box, b.maxcl, b.lstate);
+    if (c.natom <= SMALL_T) {
+        // one atom per thread: 648 sites 1480 -> 1300 us per 24 steps, 864 sites
+        // 1475 -> 1410 per 40.  Beyond, one workgroup takes longer than four
+        // launches (3,009 sites: 1018 -> 1100 us per 10 steps; 2,997 sites that
+        // build every step: 763 -> 990 per 6)
+        hipLaunchKernelGGL(k_build_small, dim3(1), dim3(SMALL_T), 0, c.stream, c.natom, nslot, x,
+                           y, z, c.atom_site, c.atom_mol, c.sites, c.mols, c.reps, fx, fy, fz,
+                           b.atom_x0, b.ncl_total, b.maxcl, b.slot_orig, b.slot_info, b.slot_w64,
+                           b.slot_x64, b.slot_off, b.slot_par, b.cl_center, b.cl_ext, b.cl_box,
+                           b.fslot, b.atom_cell, b.atom_slot, b.atom_wz, b.cell_count,
+                           b.cell_start, b.cell_members, b.col_cell0, b.col_cl0, b.cl_col,
+                           b.col_rep, b.atom_gslot, b.ncell, b.ncol, c.status, b.lstate,
+                           half_skin2, force, b.half, b.hist);
+    } else {
+        // one-wave workgroups: the check is a short chain of dependent loads,
+        // which more, smaller workgroups spread over more CUs (0.9 us per step)
+        hipLaunchKernelGGL(k_list_check, dim3((std::max(c.natom, nslot) + 63) / 64), dim3(64), 0,
+                           c.stream, c.natom, nslot, x, y, z, c.atom_site, c.sites, fx, fy, fz,
+                           b.atom_x0, b.ncl_total, b.maxcl, b.slot_orig, b.slot_w64, b.cl_center,
+                           b.slot_x64, b.slot_off, b.cl_box, b.fslot, b.lstate, half_skin2, force,
+                           b.half, b.hist);
+        // the last binning workgroup scans the cells.  1024 threads scan, and
+        // arrive, faster where there are many (8,813 cells: 24.7 against 34.3 us;
+        // 6,144: 18.3 against 25.2); at 1,331 cells both take 13.0, and smaller
+        // systems would leave CUs idle while they bin.  But a workgroup of 16 waves
+        // also waits for a CU free of the side stream's work on the steps that
+        // build nothing (98,304 sites: 125 us behind the structure factors), so
+        // they are for calls that always build.
+        auto bin = [&](auto kernel, int nt) {
+            hipLaunchKernelGGL(kernel, dim3((c.natom + nt - 1) / nt), dim3(nt), 0, c.stream, c.natom,
+                               x, y, z, c.atom_site, c.atom_mol, c.sites, c.mols, c.reps, b.atom_cell,
+                               b.atom_slot, b.atom_wz, b.cell_count, fx, fy, fz, b.atom_gslot,
+                               c.status, b.lstate, b.ncell, b.ncol, b.cell_start, b.col_cell0,
+                               b.col_cl0, b.cl_col, b.ncl_total, b.maxcl, b.bin_ctr);
+        };
+        if (b.ncell > 2048 && (force || half_skin2 == 0.0))
+            bin(k_bin_scan<1024>, 1024);
+        else
+            bin(k_bin_scan<256>, 256);
+        hipLaunchKernelGGL(k_scatter, dim3(gA), dim3(T), 0, c.stream, c.natom, b.atom_cell,
+                           b.atom_slot, b.cell_start, b.cell_members, b.lstate);
+        // threads for 1.25 times the mean column, up to 1024 (a column of a long
+        // box holds thousands of atoms): a workgroup much larger than its column
+        // idles (70,508 atoms in 1,600 columns: 28.6 us with 1024 threads, 13.5
+        // with 64), and where no list is built it still waits for a CU with 16
+        // free waves.
+        int tp = 64;
+        while (tp < 1024 && (double)tp * b.ncol < 1.25 * c.natom) tp *= 2;
+        hipLaunchKernelGGL(k_place_bbox, dim3(b.ncol), dim3(tp), 0, c.stream, b.ncol, x, y, z,
+                           b.atom_cell, b.atom_wz, b.cell_start, b.cell_members, c.atom_mol,
+                           c.atom_site, c.mols, c.reps, b.col_cell0, b.col_cl0, b.col_rep,
+                           b.ncl_total, b.slot_orig, b.slot_info, b.slot_x64, b.slot_w64, b.atom_x0,
+                           b.atom_gslot, c.sites, b.slot_off, b.slot_par, b.cl_center, b.cl_ext,
+                           b.cl_box, b.maxcl, b.lstate);
+    }
     int gP = (b.maxcl * 64 + T - 1) / T;
     hipLaunchKernelGGL(k_plist, dim3(gP), dim3(T), 0, c.stream, b.ncl_total, b.maxcl, b.cl_col,
                        b.col_cl0, b.col_rep, b.col_cell0, b.cell_start, c.reps, b.cl_center,

@@ -1,7 +1,8 @@
 """The list build's launch shapes: binning workgroups of 256 and 1024 threads
 (up to 2,048 cells and above) and placing workgroups of 64 to 1024 threads (by
 atoms per column), from the cells a system is given; the pairs found are the
-oracle's, exactly, on a first build and on a rebuild after every atom moved."""
+oracle's, exactly.  And the build of up to 1,024 atoms by one workgroup, on a
+first build, on reuse of the list and on a rebuild."""
 import numpy as np
 import pytest
 
@@ -27,4 +28,41 @@ def test_pairs_of_every_launch_shape(cell_atoms):
         for k in ("n_lj_pairs", "lj_pair_hash"):
             assert u[k] == t[k], (k, u[k], t[k])
         assert np.linalg.norm(g - f) <= 1e-12 * np.linalg.norm(f)
+    eng.close()
+
+
+SMALL = {
+    "water-1": lambda: [configs.water_box(n_side=1, L=8.0, rc=3.9, kappa=0.5, nmol=1, seed=2)],
+    "water-341": lambda: [configs.water_box(n_side=7, L=21.7, rc=7.0, nmol=341, seed=2)],  # 1,023
+    "water-342": lambda: [configs.water_box(n_side=7, L=21.7, rc=7.0, nmol=342, seed=2)],  # 1,026
+    "batch": lambda: [configs.water_box(n_side=5, L=15.5, rc=7.0, nmol=n, seed=n)
+                      for n in (1, 125, 30)],
+    "ghosts": lambda: [configs.mixture_box(n_water=40, n_co=30, L=18.0, rc=8.5, water4=True)],
+}
+
+
+@pytest.mark.parametrize("name", list(SMALL))
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_pairs_of_small_systems(name, precision):
+    systems = [system_of(rd) for rd in SMALL[name]()]
+    print(f"{name} {precision}", flush=True)
+    eng = Engine.replicas(systems, precision=precision)
+    skin = 0.6 / systems[0].params["sigma_base"]
+    eng.set_list_skin(skin)
+    rng = np.random.default_rng(5)
+    # from the first positions: none, every atom by less than half the skin
+    # (reuse), by more (rebuild)
+    unit = [rng.uniform(-1.0, 1.0, (3, s.natom)) / np.sqrt(3.0) for s in systems]
+    for d in (0.0, 0.45 * skin, 0.9 * skin):
+        xs = [np.stack([s.xx, s.yy, s.zz]) + d * u for s, u in zip(systems, unit)]
+        g, terms = eng.frclong(*eng.pack(xs))
+        terms = [terms] if isinstance(terms, dict) else terms
+        for s, x, f, u in zip(systems, xs, eng.unpack(g), terms):
+            fo, to = Oracle(s).frclong(*x)
+            if precision == "fp64":
+                for k in ("n_lj_pairs", "n_elec_pairs", "lj_pair_hash", "elec_pair_hash"):
+                    assert u[k] == to[k], (k, u[k], to[k])
+            # FP32 pair terms of the mixed kernel: 6e-8 each, with cancellation
+            tol = 1e-12 if precision == "fp64" else 2e-5
+            assert np.linalg.norm(f - fo) <= tol * np.linalg.norm(fo)
     eng.close()
