@@ -422,7 +422,7 @@ struct SlotForces {
 };
 struct FinAtoms {
     double *fx, *fy, *fz;
-    const double* frec;  // (3, natom)
+    const double* frec;  // (3, natom), or null: no such forces
     Kick K;
     int natom;
     SlotForces S;
@@ -434,7 +434,8 @@ void launch_intra(const LaunchCtx& c, const SpeciesDev* species,
                   const double* z, double* fx, double* fy, double* fz,
                   double* epart, double* gq = nullptr, double* ge = nullptr,
                   double* gs = nullptr, const double* frec = nullptr,
-                  const Kick* kick = nullptr, bool zero_first = false);
+                  const Kick* kick = nullptr, bool zero_first = false,
+                  const SlotForces* slots = nullptr);
 // (zero_first: each molecule's thread sets its atoms' fx..fz to zero before
 // adding, so fx..fz need no clearing pass)
 // fx += (slot forces, when given) + frec ((3, N) reciprocal-space forces),

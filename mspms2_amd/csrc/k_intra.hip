@@ -269,7 +269,7 @@ __global__ void __launch_bounds__(64 * NW) k_intra_tw(
     int nmol, const MolDev* __restrict__ mols, const RepDev* __restrict__ reps,
     const SiteDev* __restrict__ sites, const TermDev* __restrict__ terms,
     const double* __restrict__ x, const double* __restrict__ y, const double* __restrict__ z,
-    double* fx, double* fy, double* fz, double* epart, Kick K, int zero_first) {
+    double* fx, double* fy, double* fz, double* epart, Kick K, int zero_first, SlotForces S) {
     __shared__ double sf[3][NW][64];   // a term's force on its first site
     __shared__ double le[4][NW][64];
     __shared__ int pr[NW][64];         // a term's sites (0xff: none) and is_long
@@ -343,6 +343,7 @@ __global__ void __launch_bounds__(64 * NW) k_intra_tw(
         const int i = base + w;
         double ax = zero_first ? 0.0 : fx[i], ay = zero_first ? 0.0 : fy[i],
                az = zero_first ? 0.0 : fz[i];
+        fold_slot(S, i, ax, ay, az);
 #pragma unroll
         for (int c = 0; c < NW; c++) {
             const int p = pr[c][mi];
@@ -543,9 +544,9 @@ __global__ void __launch_bounds__(FIN_T) k_finalize(
             const int a = Ra.atom0 + i;
             double ax = A.fx[a], ay = A.fy[a], az = A.fz[a];
             fold_slot(A.S, a, ax, ay, az);
-            A.fx[a] = ax + A.frec[a];
-            A.fy[a] = ay + A.frec[n + a];
-            A.fz[a] = az + A.frec[2 * n + a];
+            A.fx[a] = A.frec ? ax + A.frec[a] : ax;
+            A.fy[a] = A.frec ? ay + A.frec[n + a] : ay;
+            A.fz[a] = A.frec ? az + A.frec[2 * n + a] : az;
             if (A.K.vx) kick_atom(A.K, a, A.fx, A.fy, A.fz);
         }
     }
@@ -979,15 +980,19 @@ void launch_grad_sites(const LaunchCtx& c, const SpeciesDev* species, const int4
 void launch_intra(const LaunchCtx& c, const SpeciesDev* species, const TermDev* terms,
                   const double* x, const double* y, const double* z, double* fx, double* fy,
                   double* fz, double* epart, double* gq, double* ge, double* gs,
-                  const double* frec, const Kick* kick, bool zero_first) {
+                  const double* frec, const Kick* kick, bool zero_first,
+                  const SlotForces* slots) {
     int g = (c.nmol + 255) / 256;
     const Kick K = kick ? *kick : Kick{};
+    const SlotForces S = slots ? *slots : SlotForces{};
+    const int most = std::max(c.max_mol_atoms, c.max_mol_intra);
+    // the kernel by terms adds the slot-ordered pair forces itself
+    if (S.f && (gq || frec || most > 6)) launch_fold_slots(c, S, fx, fy, fz);
     auto by_term = [&](auto kernel, int nw) {
         hipLaunchKernelGGL(kernel, dim3((c.nmol + 63) / 64), dim3(64 * nw), 0, c.stream, c.nmol,
                            c.mols, c.reps, c.sites, terms, x, y, z, fx, fy, fz, epart, K,
-                           zero_first ? 1 : 0);
+                           zero_first ? 1 : 0, S);
     };
-    const int most = std::max(c.max_mol_atoms, c.max_mol_intra);
     if (!gq && !frec && most <= 3)
         by_term(k_intra_tw<3>, 3);
     else if (!gq && !frec && most <= 4)
