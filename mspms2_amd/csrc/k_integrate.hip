@@ -416,7 +416,7 @@ struct NptInner {
     int nrep;
 };
 
-template <int NW, bool NPT>
+template <int NW, int NA, bool NPT>
 __global__ void __launch_bounds__(64 * NW) k_respa_inner_tw(
     int nmol, const MolDev* __restrict__ mols, const SpeciesDev* __restrict__ species,
     const TermDev* __restrict__ terms, const SiteDev* __restrict__ sites, double* x, double* y,
@@ -430,8 +430,8 @@ __global__ void __launch_bounds__(64 * NW) k_respa_inner_tw(
         if (r < NB.nrep) npt_box(NB.reps[r], NB.st[r], delts, nstep_inner);
         return;
     }
-    __shared__ double lx[NW * 64], ly[NW * 64], lz[NW * 64];
-    __shared__ double cfx[NW][NW * 64], cfy[NW][NW * 64], cfz[NW][NW * 64];
+    __shared__ double lx[NA * 64], ly[NA * 64], lz[NA * 64];
+    __shared__ double cfx[NW][NA * 64], cfy[NW][NA * 64], cfz[NW][NA * 64];
     __shared__ double le[NW][5][64];
     const int w = threadIdx.x >> 6, mi = threadIdx.x & 63;
     const int m = blockIdx.x * 64 + mi;
@@ -489,7 +489,7 @@ __global__ void __launch_bounds__(64 * NW) k_respa_inner_tw(
     const bool stores = term && ((T.kind == TERM_BOND && T.type == MSPMS_BOND_HARMONIC) ||
                                  (T.kind == TERM_ANGLE && T.type == MSPMS_ANGLE_HARMONIC));
 #pragma unroll
-    for (int k = 0; k < NW; k++) {
+    for (int k = 0; k < NA; k++) {
         cfx[w][k * 64 + mi] = 0.0;
         cfy[w][k * 64 + mi] = 0.0;
         cfz[w][k * 64 + mi] = 0.0;
@@ -521,7 +521,7 @@ __global__ void __launch_bounds__(64 * NW) k_respa_inner_tw(
         __syncthreads();  // the positions are in; every copy has been read
         if (!stores && ll > 0) {
 #pragma unroll
-            for (int k = 0; k < NW; k++) {
+            for (int k = 0; k < NA; k++) {
                 cfx[w][k * 64 + mi] = 0.0;
                 cfy[w][k * 64 + mi] = 0.0;
                 cfz[w][k * 64 + mi] = 0.0;
@@ -786,8 +786,9 @@ void launch_respa_inner(const LaunchCtx& c, const SpeciesDev* species, const Ter
                        c.nmol, c.mols, species, terms, c.sites, x, y, z, vx, vy, vz, fxl, fyl,   \
                        fzl, fxs, fys, fzs, deltby2, delts, deltsby2, nstep_inner, epart,        \
                        c.status, c.rep_delt, W, SN)
-#define RESPA_TW(NW)                                                                         \
-    hipLaunchKernelGGL((k_respa_inner_tw<NW, false>), dim3((c.nmol + 63) / 64), dim3(64 * NW), 0, \
+#define RESPA_TW(NW, NA)                                                                     \
+    hipLaunchKernelGGL((k_respa_inner_tw<NW, NA, false>), dim3((c.nmol + 63) / 64),              \
+                       dim3(64 * NW), 0,                                                          \
                        c.stream, c.nmol, c.mols, species, terms, c.sites, x, y, z, vx, vy, vz,    \
                        fxl, fyl, fzl, fxs, fys, fzs, deltby2, delts, deltsby2, nstep_inner,       \
                        epart, c.status, c.rep_delt, W, SN, NptInner{})
@@ -805,9 +806,11 @@ void launch_respa_inner(const LaunchCtx& c, const SpeciesDev* species, const Ter
     } else if (c.max_mol_atoms <= 1) {
         RESPA_TPM(1, 1);  // one lane per single-site molecule
     } else if (c.max_mol_atoms <= 3 && c.max_mol_terms <= 3) {
-        RESPA_TW(3);  // e.g. flexible three-site water: one term per wave
+        RESPA_TW(3, 3);  // e.g. flexible three-site water: one term per wave
     } else if (c.max_mol_atoms <= 4 && c.max_mol_terms <= 4) {
-        RESPA_TW(4);
+        RESPA_TW(4, 4);
+    } else if (c.max_mol_atoms <= 4 && c.max_mol_terms <= 6) {
+        RESPA_TW(6, 4);  // e.g. four united atoms: three bonds, two angles, a dihedral
     } else if (c.max_mol_atoms <= 4) {
         RESPA_TPM(4, 4);
     } else if (c.max_mol_atoms <= 8) {
@@ -840,9 +843,10 @@ bool launch_npt_inner_loop(const LaunchCtx& c, const TermDev* terms, RepDev* rep
         return true;
     };
     const int most = std::max(c.max_mol_atoms, c.max_mol_terms);
-    if (most <= 1) return run(k_respa_inner_tw<1, true>, 1);
-    if (most <= 3) return run(k_respa_inner_tw<3, true>, 3);
-    if (most <= 4) return run(k_respa_inner_tw<4, true>, 4);
+    if (most <= 1) return run(k_respa_inner_tw<1, 1, true>, 1);
+    if (most <= 3) return run(k_respa_inner_tw<3, 3, true>, 3);
+    if (most <= 4) return run(k_respa_inner_tw<4, 4, true>, 4);
+    if (c.max_mol_atoms <= 4 && most <= 6) return run(k_respa_inner_tw<6, 4, true>, 6);
     return false;
 }
 

@@ -1,6 +1,7 @@
 """The NPT step (k_npt.hip, and the inner loop in one launch of
 k_integrate.hip) on every path that its dispatch takes -- single sites,
-molecules of up to three and four sites and terms, larger ones -- at the edges
+molecules of up to three and four sites and terms, four sites and
+six terms, larger ones -- at the edges
 of their workgroups and where a replica has more atoms than its workgroup
 keeps in registers (4,096), against the CPU restatement of npt_respa
 (tests/md_cpu.py).  Two steps in FP64 with the bounds of test_gpu_md.py."""
@@ -22,7 +23,9 @@ CASES = {
     "water-64": lambda: [_water(64)],
     "water-batch": lambda: [_water(1), _water(65), _water(125)],
     "chain-65": lambda: [_chain(65)],
-    "butane-64": lambda: [configs.butane_box(nmol=64)],     # 6 terms: a launch per inner step
+    "butane-64": lambda: [configs.butane_box(nmol=64)],
+    "butane-65": lambda: [configs.butane_box(nmol=65)],
+    "zoo-43": lambda: [configs.bonded_zoo(nmole=43)],       # a launch per inner step
 }
 
 
