@@ -533,7 +533,8 @@ __global__ void __launch_bounds__(64 * NW) k_respa_inner_tw(
             double u = 0.0, v = 0.0;
             int sing = 0;
             const int cls =
-                bonded_term_inner(T, mi, lx, ly, lz, cfx[w], cfy[w], cfz[w], &u, &v, &sing, 64);
+                bonded_term_inner(T, mi, lx, ly, lz, cfx[w], cfy[w], cfz[w], &u, &v, &sing, 64,
+                                  ll + 1 == nstep_inner);  // the last step's energies are read
             if (sing) atomicOr(&st->flags, ST_SINGULAR);
             e[cls] += u;
             vir += v;
