@@ -171,11 +171,16 @@ __global__ void __launch_bounds__(64 * WPC, 4) k_pair(
         const double ec = erfc_exp64(x, xl, &ex);
         const double cq = Cqi * B.p.w;
         double ug, f;  // energy per charge product, force / r
-        if (ELEC == MSPMS_ELEC_EWALD) {
+        if (ELEC == MSPMS_ELEC_EWALD)
             ug = ri * ec;
+        else
+            ug = fma(ec, ri, fma(R.wvc2, (r - R.rc_el) + rl, R.wvc1));
+        // sites on one point: an infinite energy and, as in the reference, no
+        // force (everything above is NaN there)
+        if (rsq == 0.0) ug = __builtin_huge_val();
+        if (ELEC == MSPMS_ELEC_EWALD) {
             f = cq * fma(ri * x * ex, 1.1283791670955126, ug) * (ri * ri);
         } else {
-            ug = fma(ec, ri, fma(R.wvc2, (r - R.rc_el) + rl, R.wvc1));
             f = cq * ri * (fma(ec, ri, R.wfc1 * ex) * ri + R.wfc2);
             vir += f * rsq;
         }

@@ -119,15 +119,13 @@ __device__ inline double rcp_nr(double x) {
     return fma(y, fma(-x, y, 1.0), y);
 }
 
-// 1 / sqrt(x) within an ulp (infinity at 0)
+// 1 / sqrt(x) within an ulp, x > 0 (NaN at 0)
 __device__ inline double rsqrt_fma(double x) {
-    const double y0 = __builtin_amdgcn_rsq(x);
-    double y = y0;
+    double y = __builtin_amdgcn_rsq(x);
     double h = 0.5 * x * y;
     y = fma(y, fma(-h, y, 0.5), y);
     h = 0.5 * x * y;
-    y = fma(y, fma(-h, y, 0.5), y);
-    return x == 0.0 ? y0 : y;
+    return fma(y, fma(-h, y, 0.5), y);
 }
 
 // erfc(x) and exp(-x^2) for x >= 0 without a branch: erfc(x) = exp(-x^2)

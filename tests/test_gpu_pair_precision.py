@@ -14,6 +14,7 @@ from mspms2_amd import abi
 from mspms2_amd.engine import Engine
 from mspms2_amd.runio import RunDir, RunInput, Site, SpeciesSpec
 from mspms2_amd.system import System
+from oracle.oracle import Oracle
 
 pytestmark = pytest.mark.gpu
 
@@ -102,3 +103,21 @@ def test_pair_terms_against_40_digits(elec):
     rms = [float(np.sqrt(np.mean(np.square(e)))) for e in (eu, ef) if e]
     print(f"RMS relative error {elec}: " + ", ".join(f"{v:.2e}" for v in rms), flush=True)
     assert max(rms) <= 4e-16, rms
+
+
+@pytest.mark.parametrize("elec", ["ewald", "wolf"])
+def test_sites_on_one_point(elec):
+    """Two charged sites on one point: the energy is infinite, with the sign of
+    the charges' product, as the reference's C q q / r gives it (a sampling
+    program rejects on it); the force has no value."""
+    for q in ((1.0, -1.0), (1.0, 0.5)):
+        s = ions([[3.0, 4.0, 5.0], [3.0, 4.0, 5.0]], elec, q)
+        _, want = Oracle(s).frclong()
+        print(f"case coincident {elec} {q}", flush=True)
+        eng = Engine(s, precision="fp64")
+        _, t = eng.frclong()
+        eng.close()
+        assert want["ureal"] == np.copysign(np.inf, q[0] * q[1])
+        assert t["n_elec_pairs"] == want["n_elec_pairs"] == 1
+        for k in ("ureal", "uelec", "uinter", "virial_inter"):
+            assert np.array_equal(t[k], want[k], equal_nan=True), (k, t[k], want[k])
