@@ -219,11 +219,6 @@ struct mspms_ctx {
     std::vector<long> prof_n;          // recorded launches per group
     bool capturing = false;            // no event records inside a capture
 
-    // one RESPA outer step captured as a graph (mspms_vver_run_device),
-    // valid for the argument set in gkey until the next build
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t graph_exec = nullptr;
-    int graph_kind = -1;                 // GRAPH_*: what the cached graph runs
 
     // batched HMC chains (mspms_hmc_init)
     DevBuf<RanmarDev> d_rng;
@@ -259,33 +254,46 @@ struct mspms_ctx {
                    st == o.st && uk == o.uk && delt == o.delt && nstep_inner == o.nstep_inner &&
                    per == o.per;
         }
-    } gkey{};
+    };
+    // device runs captured as graphs, one step (or move) and RUN_GRAPH_STEPS
+    // steps, each valid for its kind and arguments until the next build
+    struct Graph {
+        hipGraph_t graph = nullptr;
+        hipGraphExec_t exec = nullptr;
+        int kind = -1;  // GRAPH_*
+        GraphKey key{};
+    } graphs[2];
 };
 
 namespace {
 
+void drop_graph(mspms_ctx::Graph& g) {
+    if (g.exec) (void)hipGraphExecDestroy(g.exec);
+    if (g.graph) (void)hipGraphDestroy(g.graph);
+    g = mspms_ctx::Graph{};
+}
+
 void drop_graph(mspms_ctx* c) {
-    if (c->graph_exec) (void)hipGraphExecDestroy(c->graph_exec);
-    if (c->graph) (void)hipGraphDestroy(c->graph);
-    c->graph_exec = nullptr;
-    c->graph = nullptr;
+    for (auto& g : c->graphs) drop_graph(g);
 }
 
 enum { GRAPH_VVER = 0, GRAPH_HMC = 1, GRAPH_NVT = 2, GRAPH_NPT = 3 };
 
-// Makes the cached graph the capture of enqueue(stream) for (kind, key),
-// capturing it again when either differs.
+// Makes the cached graph of key.per steps the capture of enqueue(stream),
+// key.per times, for (kind, key), capturing it again when either differs.
 template <typename F>
 int ensure_graph(mspms_ctx* c, hipStream_t s, int kind, const mspms_ctx::GraphKey& key,
                  F&& enqueue) {
-    if (c->graph_exec && key == c->gkey && c->graph_kind == kind) return 0;
-    drop_graph(c);
+    mspms_ctx::Graph& G = c->graphs[key.per > 1];
+    if (G.exec && key == G.key && G.kind == kind) return 0;
+    drop_graph(G);
     // the capture stream must not have work in flight from the caller
     HIPC(hipStreamSynchronize(s));
     HIPC(hipStreamSynchronize(c->stream));
     c->capturing = true;
     HIPC(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-    int rc = enqueue(c->stream);
+    int rc = 0;
+    for (int q = 0; q < key.per && !rc; q++) rc = enqueue(c->stream);
     hipGraph_t g = nullptr;
     hipError_t e = hipStreamEndCapture(c->stream, &g);
     c->capturing = false;
@@ -294,14 +302,14 @@ int ensure_graph(mspms_ctx* c, hipStream_t s, int kind, const mspms_ctx::GraphKe
         return rc;
     }
     if (e != hipSuccess) return fail(MSPMS_EIO, "graph capture: %s", hipGetErrorString(e));
-    c->graph = g;
-    e = hipGraphInstantiate(&c->graph_exec, g, nullptr, nullptr, 0);
+    G.graph = g;
+    e = hipGraphInstantiate(&G.exec, g, nullptr, nullptr, 0);
     if (e != hipSuccess) {
-        drop_graph(c);
+        drop_graph(G);
         return fail(MSPMS_EIO, "graph instantiate: %s", hipGetErrorString(e));
     }
-    c->gkey = key;
-    c->graph_kind = kind;
+    G.key = key;
+    G.kind = kind;
     return 0;
 }
 
@@ -1606,20 +1614,36 @@ int enqueue_vver(mspms_ctx* c, double* pos, double* vel, double* fl, double* fs,
     return 0;
 }
 
-// Steps per captured graph of a device run.  Four steps in one graph drop
-// three of the four graph boundaries per four steps (0.6 us per step at the
-// 12,288-site water step of ~97 us); the steps that four does not divide are
-// enqueued one by one, at about 16 us more each (6 NVT steps of 12,288
-// sites: 943 us as one graph of four and two steps, 910 as six graphs).  So
-// short runs take the largest count up to four that leaves none over, and
-// runs of 64 steps or more, where three such steps are made up for, take four.
+// Steps of the longer of a device run's two graphs.  Four steps in one graph
+// drop three of the four graph boundaries per four steps (0.6 us per step at
+// the 12,288-site water step of ~97 us); the steps that four does not divide
+// replay a graph of one step (enqueued kernel by kernel they take about 16 us
+// more each: 6 NVT steps of 12,288 sites 943 us, 910 as six graphs).  Both
+// graphs stay, whatever length the next run has: a program that runs 10, 9
+// and 8 steps in turn captures each once.
 constexpr int RUN_GRAPH_STEPS = 4;
 
-int run_graph_steps(int nsteps) {
-    if (nsteps >= 16 * RUN_GRAPH_STEPS) return RUN_GRAPH_STEPS;
-    int per = RUN_GRAPH_STEPS;
-    while (per > 1 && (nsteps < per || nsteps % per)) per--;
-    return per;
+// How many steps of a run go by graphs of RUN_GRAPH_STEPS: short runs that need
+// the graph of one step anyway take that alone, since capturing the longer
+// one as well costs a first run of 10 steps about 70 us (3,009 sites) and
+// saves each later one about 4.
+int long_graph_steps(int nsteps) {
+    if (nsteps < 4 * RUN_GRAPH_STEPS && nsteps % RUN_GRAPH_STEPS) return 0;
+    return nsteps - nsteps % RUN_GRAPH_STEPS;
+}
+
+// the graphs that nsteps steps need
+template <typename F>
+int ensure_run_graphs(mspms_ctx* c, hipStream_t s, int kind, mspms_ctx::GraphKey key, int nsteps,
+                      F&& enqueue) {
+    const int by_long = long_graph_steps(nsteps);
+    int rc = 0;
+    for (int per : {RUN_GRAPH_STEPS, 1}) {
+        key.per = per;
+        if (!rc && (per > 1 ? by_long > 0 : by_long < nsteps))
+            rc = ensure_graph(c, s, kind, key, enqueue);
+    }
+    return rc;
 }
 
 // Closes the finalize gate for a run of device steps whose terms nobody reads
@@ -1890,10 +1914,10 @@ extern "C" int mspms_vver_step_device(mspms_ctx* c, double* pos, double* vel, do
     return enqueue_vver(c, pos, vel, fl, fs, delt, nstep_inner, lterms, sterms, ukin, s);
 }
 
-// nsteps RESPA outer steps; with use_graph a few steps (run_graph_steps) are
-// captured once as a HIP graph (on the context stream) and replayed on
-// `stream`, the steps left over enqueued directly.  Optional histories receive each step's terms (nsteps
-// * nrep entries) and kinetic energies (nsteps * nrep doubles).
+// nsteps RESPA outer steps; with use_graph graphs of RUN_GRAPH_STEPS steps and
+// of one step, captured once (on the context stream), are replayed on
+// `stream`.  Optional histories receive each step's terms (nsteps * nrep
+// entries) and kinetic energies (nsteps * nrep doubles).
 extern "C" int mspms_vver_run_device(mspms_ctx* c, double* pos, double* vel, double* fl,
                                      double* fs, double delt, int nstep_inner, int nsteps,
                                      mspms_long_terms* lterms, mspms_short_terms* sterms,
@@ -1907,16 +1931,10 @@ extern "C" int mspms_vver_run_device(mspms_ctx* c, double* pos, double* vel, dou
     HIPC(hipSetDevice(c->device));
     hipStream_t s = stream ? (hipStream_t)stream : c->stream;
     const int nr = c->nrep;
-    const int per = run_graph_steps(nsteps);
     if (use_graph) {
-        mspms_ctx::GraphKey k{pos, vel, fl, fs, lterms, sterms, ukin, delt, nstep_inner, per};
-        int rc = ensure_graph(c, s, GRAPH_VVER, k, [&](hipStream_t cs) {
-            for (int q = 0; q < per; q++) {
-                int rq = enqueue_vver(c, pos, vel, fl, fs, delt, nstep_inner, lterms, sterms,
-                                      ukin, cs);
-                if (rq) return rq;
-            }
-            return 0;
+        mspms_ctx::GraphKey k{pos, vel, fl, fs, lterms, sterms, ukin, delt, nstep_inner};
+        int rc = ensure_run_graphs(c, s, GRAPH_VVER, k, nsteps, [&](hipStream_t cs) {
+            return enqueue_vver(c, pos, vel, fl, fs, delt, nstep_inner, lterms, sterms, ukin, cs);
         });
         if (rc) return rc;
     }
@@ -1956,17 +1974,16 @@ extern "C" int mspms_vver_run_device(mspms_ctx* c, double* pos, double* vel, dou
         hist_off.on = true;
     }
     for (int t = 0; t < nsteps;) {
-        // a graph of `per` steps while that many remain, then single steps
-        const bool grp = use_graph && nsteps - t >= per;
-        const int adv = grp ? per : 1;
+        const bool grp = use_graph && t < long_graph_steps(nsteps);
+        const int adv = grp ? RUN_GRAPH_STEPS : 1;
         if (gate && t + adv >= nsteps) {
             // the launch that holds the last step reduces its terms (the
             // other steps of a graph reduce theirs too: the last one wins)
             HIPC(fin.set(true));
         }
         t += adv;
-        if (grp) {
-            HIPC(hipGraphLaunch(c->graph_exec, s));
+        if (use_graph) {
+            HIPC(hipGraphLaunch(c->graphs[grp].exec, s));
         } else {
             int rc = enqueue_vver(c, pos, vel, fl, fs, delt, nstep_inner, lterms, sterms, ukin, s);
             if (rc) return rc;
@@ -2153,7 +2170,7 @@ extern "C" int mspms_hmc_run_device(mspms_ctx* c, double* pos, double* vel, doub
                                     ukin, cs);
         });
         if (rc) return rc;
-        for (int m = 0; m < nmove; m++) HIPC(hipGraphLaunch(c->graph_exec, s));
+        for (int m = 0; m < nmove; m++) HIPC(hipGraphLaunch(c->graphs[0].exec, s));
         return 0;
     }
     for (int m = 0; m < nmove; m++) {
@@ -2363,27 +2380,22 @@ extern "C" int mspms_nvt_run_device(mspms_ctx* c, double* pos, double* vel, doub
     hipStream_t s = stream ? (hipStream_t)stream : c->stream;
     // graphs of several steps, and the terms of the last step only, as in
     // the NVE run
-    const int per = run_graph_steps(nsteps);
     if (use_graph) {
-        mspms_ctx::GraphKey k{pos, vel, fl, fs, lterms, sterms, ukin, delt, nstep_inner, per};
-        int rc = ensure_graph(c, s, GRAPH_NVT, k, [&](hipStream_t cs) {
-            for (int q = 0; q < per; q++) {
-                int rq = enqueue_nvt(c, pos, vel, fl, fs, delt, nstep_inner, lterms, sterms, ukin,
-                                     cs);
-                if (rq) return rq;
-            }
-            return 0;
+        mspms_ctx::GraphKey k{pos, vel, fl, fs, lterms, sterms, ukin, delt, nstep_inner};
+        int rc = ensure_run_graphs(c, s, GRAPH_NVT, k, nsteps, [&](hipStream_t cs) {
+            return enqueue_nvt(c, pos, vel, fl, fs, delt, nstep_inner, lterms, sterms, ukin, cs);
         });
         if (rc) return rc;
     }
+    // the terms of the last step only, as in the NVE run
     FinGate fin{c, s};
     if (nsteps > 1) HIPC(fin.set(false));
     for (int t = 0; t < nsteps;) {
-        const bool grp = use_graph && nsteps - t >= per;
-        t += grp ? per : 1;
+        const bool grp = use_graph && t < long_graph_steps(nsteps);
+        t += grp ? RUN_GRAPH_STEPS : 1;
         if (fin.closed && t >= nsteps) HIPC(fin.set(true));
-        if (grp) {
-            HIPC(hipGraphLaunch(c->graph_exec, s));
+        if (use_graph) {
+            HIPC(hipGraphLaunch(c->graphs[grp].exec, s));
         } else {
             int rc = enqueue_nvt(c, pos, vel, fl, fs, delt, nstep_inner, lterms, sterms, ukin, s);
             if (rc) return rc;
@@ -2549,7 +2561,7 @@ extern "C" int mspms_npt_run_device(mspms_ctx* c, double* pos, double* vel, doub
             return enqueue_npt(c, pos, vel, fl, fs, delt, nstep_inner, lterms, sterms, ukin, cs);
         });
         if (rc) return rc;
-        for (int t = 0; t < nsteps; t++) HIPC(hipGraphLaunch(c->graph_exec, s));
+        for (int t = 0; t < nsteps; t++) HIPC(hipGraphLaunch(c->graphs[0].exec, s));
         return 0;
     }
     for (int t = 0; t < nsteps; t++) {

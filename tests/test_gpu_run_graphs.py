@@ -1,5 +1,5 @@
-"""NVE and NVT device runs whose step counts give graphs of one to four steps,
-steps left over, and terms reduced for the last step only: the same state and
+"""NVE and NVT device runs whose step counts give graphs of one and four steps,
+both, and terms reduced for the last step only: the same state and
 the same terms as one-step calls without graphs.  FP64, whose sums all have a
 fixed order, so the two differ by nothing."""
 import numpy as np
@@ -45,4 +45,69 @@ def test_runs_equal_single_steps(kind):
         for graph in (True, False):
             for g, w in zip(run([n], graph), want):
                 assert torch.equal(g.view(torch.int64), w.view(torch.int64))
+    eng.close()
+
+
+def _waits(stream, calls):
+    """Whether calls() waits for work that lies ahead of it on the stream (some
+    400 ms of matrix products)."""
+    import torch
+    with torch.cuda.stream(stream):
+        big = torch.zeros(8192, 8192, device="cuda:0")
+        out = torch.mm(big, big)
+        torch.cuda.synchronize()
+        for _ in range(60):
+            torch.mm(big, big, out=out)
+        done = torch.cuda.Event()
+        done.record()
+    calls()
+    waited = done.query()
+    torch.cuda.synchronize()
+    return waited
+
+
+@pytest.mark.parametrize("kind", ["nve", "nvt"])
+def test_changing_lengths_capture_once(kind):
+    """Runs of changing lengths on the same buffers: once every length has been
+    seen, a call waits for nothing (a capture waits for the stream it is to be
+    replayed on), and the states are those of one-step calls."""
+    import torch
+    s = system_of(configs.water_box(n_side=3, L=9.4, rc=4.5, kappa=0.6, kmax=4, ksqmax=16, seed=8))
+    v0 = np.random.default_rng(2).standard_normal((3, s.natom)) * np.sqrt(s.treq / s.masses())
+    dev = torch.device("cuda:0")
+    t = lambda a: torch.tensor(a, dtype=torch.float64, device=dev).contiguous()  # noqa: E731
+    eng = Engine.replicas([s], precision="fp64")
+    eng.set_list_skin(0.0)
+    start = [t(a) for a in (eng.packed_positions(), v0, eng.frclong()[0], eng.frcshort()[0])]
+    bufs = [torch.empty_like(a) for a in start]
+    lt = torch.zeros(LONG_TERMS_BYTES // 8, dtype=torch.float64, device=dev)
+    st = torch.zeros(SHORT_TERMS_BYTES // 8, dtype=torch.float64, device=dev)
+    uk = torch.zeros(1, dtype=torch.float64, device=dev)
+    stream = torch.cuda.Stream()
+    call = eng.nvt_run_device if kind == "nvt" else eng.vver_run_device
+    lengths = (10, 9, 8, 3, 17)
+
+    def reset():
+        if kind == "nvt":
+            eng.nvt_set(4.0 * s.natom, 2.0 * s.natom, s.treq, 3 * s.natom - 3)
+        with torch.cuda.stream(stream):
+            for b, a in zip(bufs, start):
+                b.copy_(a)
+        torch.cuda.synchronize()
+
+    def run(parts, graph):
+        for n in parts:
+            call(*bufs, 0.25 * s.delt, 2, n, lt, st, uk, graph=graph, stream=stream.cuda_stream)
+
+    print(f"case {kind} {lengths}", flush=True)
+    reset()
+    run([1] * sum(lengths), False)
+    torch.cuda.synchronize()
+    want = [b.cpu() for b in (*bufs, lt, st, uk)]
+    reset()
+    run(lengths, True)
+    torch.cuda.synchronize()
+    for g, w in zip((*bufs, lt, st, uk), want):
+        assert torch.equal(g.cpu().view(torch.int64), w.view(torch.int64))
+    assert not _waits(stream, lambda: run(lengths, True)), "a run waited for the work ahead of it"
     eng.close()
