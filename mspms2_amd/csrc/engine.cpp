@@ -2225,15 +2225,9 @@ int enqueue_nvt(mspms_ctx* c, double* pos, double* vel, double* fl, double* fs, 
     return 0;
 }
 
-}  // namespace
-
-extern "C" int mspms_nvt_set(mspms_ctx* c, const mspms_nvt_state* st) {
-    if (!c || c->sp.empty()) return fail(MSPMS_EINVAL, "context has no system");
-    if (!st) return fail(MSPMS_EINVAL, "null argument");
-    for (int r = 0; r < c->nrep; r++)
-        if (!(st[r].qq > 0.0) || !(st[r].qqs > 0.0) || !(st[r].treq > 0.0) || st[r].nfree < 1)
-            return fail(MSPMS_EINVAL, "replica %d: qq, qqs, treq and nfree must be positive", r);
-    HIPC(hipSetDevice(c->device));
+// The NVT kernels' work lists and workspaces, which follow from the system and
+// its replicas alone.
+int make_nvt_plan(mspms_ctx* c) {
     // the workgroups of the substep kernel (by molecules, where they fit it)
     // and of the atom passes; every replica has at least one
     std::vector<int4> work[2];
@@ -2261,12 +2255,30 @@ extern "C" int mspms_nvt_set(mspms_ctx* c, const mspms_nvt_state* st) {
         (rc = c->d_nvt_blk_m.upload(blk[0], c->stream)) ||
         (rc = c->d_nvt_blk_a.upload(blk[1], c->stream)) ||
         (rc = c->d_nvt_part.ensure(2 * npart)) ||
-        (rc = c->d_nvt_scal.ensure((size_t)2 * c->nrep)) ||
-        (rc = c->d_active.upload(std::vector<int>(c->nrep, 1), c->stream)))
+        (rc = c->d_nvt_scal.ensure((size_t)2 * c->nrep)) || (rc = c->d_active.ensure(c->nrep)))
         return rc;
     c->nvt_plan = NvtPlan{c->d_nvt_work_m.p, c->d_nvt_work_a.p, c->d_nvt_blk_m.p,
                           c->d_nvt_blk_a.p,  (int)work[0].size(), (int)work[1].size(),
                           c->d_nvt_part.p,   c->d_nvt_scal.p,     npart};
+    HIPC(hipStreamSynchronize(c->stream));  // the lists have been read
+    return 0;
+}
+
+}  // namespace
+
+extern "C" int mspms_nvt_set(mspms_ctx* c, const mspms_nvt_state* st) {
+    if (!c || c->sp.empty()) return fail(MSPMS_EINVAL, "context has no system");
+    if (!st) return fail(MSPMS_EINVAL, "null argument");
+    for (int r = 0; r < c->nrep; r++)
+        if (!(st[r].qq > 0.0) || !(st[r].qqs > 0.0) || !(st[r].treq > 0.0) || st[r].nfree < 1)
+            return fail(MSPMS_EINVAL, "replica %d: qq, qqs, treq and nfree must be positive", r);
+    HIPC(hipSetDevice(c->device));
+    // (a new state of the same system leaves the buffers, and the graphs that
+    // hold them, where they are)
+    int rc;
+    if (!c->nvt_ready && (rc = make_nvt_plan(c))) return rc;
+    const std::vector<int> all(c->nrep, 1);
+    if ((rc = c->d_active.upload(all, c->stream))) return rc;
     HIPC(hipMemcpyAsync(c->d_nvt.p, st, sizeof(mspms_nvt_state) * c->nrep,
                         hipMemcpyHostToDevice, c->stream));
     HIPC(hipStreamSynchronize(c->stream));

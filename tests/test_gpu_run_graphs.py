@@ -111,3 +111,38 @@ def test_changing_lengths_capture_once(kind):
         assert torch.equal(g.cpu().view(torch.int64), w.view(torch.int64))
     assert not _waits(stream, lambda: run(lengths, True)), "a run waited for the work ahead of it"
     eng.close()
+
+
+def test_new_thermostats_keep_the_graph():
+    """mspms_nvt_set between the runs of one system: no new capture (the call
+    does not wait for work on the runs' stream), and the run starts from the new
+    state."""
+    import torch
+    s = system_of(configs.lj_fcc(ncell=4, jitter=0.04, seed=5))
+    v0 = np.random.default_rng(2).standard_normal((3, s.natom)) * np.sqrt(s.treq / s.masses())
+    dev = torch.device("cuda:0")
+    t = lambda a: torch.tensor(a, dtype=torch.float64, device=dev).contiguous()  # noqa: E731
+    eng = Engine.replicas([s], precision="fp64")
+    start = [t(eng.packed_positions()), t(v0), t(eng.frclong()[0]), torch.zeros_like(t(v0))]
+    lt = torch.zeros(LONG_TERMS_BYTES // 8, dtype=torch.float64, device=dev)
+    st = torch.zeros(SHORT_TERMS_BYTES // 8, dtype=torch.float64, device=dev)
+    uk, stream = torch.zeros(1, dtype=torch.float64, device=dev), torch.cuda.Stream()
+    bufs = [b.clone() for b in start]
+
+    def one(q):
+        eng.nvt_set(q, q, s.treq, 3 * s.natom - 3)
+        eng.nvt_run_device(*bufs, s.delt, 1, 4, lt, st, uk, stream=stream.cuda_stream)
+
+    def fresh(q):
+        for b, a in zip(bufs, start):
+            b.copy_(a)
+        torch.cuda.synchronize()
+        one(q)
+        torch.cuda.synchronize()
+        return eng.nvt_get()
+
+    print("case nvt_set between runs", flush=True)
+    first, other = fresh(100.0), fresh(7.0)
+    assert first != other and fresh(100.0) == first
+    assert not _waits(stream, lambda: one(50.0)), "nvt_set or the run after it waited"
+    eng.close()
