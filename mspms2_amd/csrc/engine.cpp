@@ -1399,6 +1399,15 @@ __global__ void k_reset_status(Status* st) {
     st->max_list = 0;
 }
 
+// A flag or counter written in stream order.  (Not a memset: the runs that use
+// it may lie in a caller's stream capture, which is to hold kernels only.)
+__global__ void k_set_int(int* p, int v) { *p = v; }
+
+hipError_t set_int(int* p, int v, hipStream_t s) {
+    hipLaunchKernelGGL(k_set_int, dim3(1), dim3(1), 0, s, p, v);
+    return hipGetLastError();
+}
+
 // The frclong terms from the partial sums; with sterms, also the frcshort
 // terms of the inner steps (ep_short) and the kinetic energy (kin).
 // gate (or null): the pass runs only while that flag is 1 (d_fin_on, which the
@@ -1647,7 +1656,7 @@ int ensure_run_graphs(mspms_ctx* c, hipStream_t s, int kind, mspms_ctx::GraphKey
 }
 
 // Closes the finalize gate for a run of device steps whose terms nobody reads
-// (written between launches, outside any capture) and opens it for the last;
+// (written between launches, outside the run's own graphs) and opens it for the last;
 // it is open again when the run returns, whatever the path.
 struct FinGate {
     mspms_ctx* c;
@@ -1655,7 +1664,7 @@ struct FinGate {
     bool closed = false;
     hipError_t set(bool open) {
         closed = !open;
-        return hipMemsetD32Async((hipDeviceptr_t)c->d_fin_on.p, open ? 1 : 0, 1, s);
+        return set_int(c->d_fin_on.p, open ? 1 : 0, s);
     }
     ~FinGate() {
         if (closed) (void)set(true);
@@ -1956,7 +1965,7 @@ extern "C" int mspms_vver_run_device(mspms_ctx* c, double* pos, double* vel, dou
     } hist_off{c, s, false};
     if (gate) HIPC(fin.set(false));
     // the overflow snapshot counts this run's steps
-    HIPC(hipMemsetAsync(c->d_snap_count.p, 0, sizeof(int), s));
+    HIPC(set_int(c->d_snap_count.p, 0, s));
     HistDev hd{};
     if (hist && nsteps > 0) {
         // every step's finalize stores its workgroup sums in slot t; the

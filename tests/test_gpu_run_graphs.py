@@ -146,3 +146,69 @@ def test_new_thermostats_keep_the_graph():
     assert first != other and fresh(100.0) == first
     assert not _waits(stream, lambda: one(50.0)), "nvt_set or the run after it waited"
     eng.close()
+
+
+def _node_types(graph):
+    """hipGraphNodeType of every node of a captured graph."""
+    import ctypes
+    path = next(line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64" in line)
+    hip, g, n = ctypes.CDLL(path), ctypes.c_void_p(graph.raw_cuda_graph()), ctypes.c_size_t()
+    assert hip.hipGraphGetNodes(g, None, ctypes.byref(n)) == 0
+    nodes, kind, out = (ctypes.c_void_p * n.value)(), ctypes.c_int(), []
+    assert hip.hipGraphGetNodes(g, nodes, ctypes.byref(n)) == 0
+    for node in nodes:
+        assert hip.hipGraphNodeGetType(ctypes.c_void_p(node), ctypes.byref(kind)) == 0
+        out.append(kind.value)
+    return out
+
+
+@pytest.mark.parametrize("kind", ["nve", "nvt"])
+def test_runs_in_a_callers_capture(kind):
+    """A run without graphs of its own, captured by the caller: kernels only (a
+    memset node can give wrong values from the second replay on), and every
+    replay, with eager work between them, leaves what the eager run leaves."""
+    import torch
+    s = system_of(configs.water_box(n_side=3, L=9.4, rc=4.5, kappa=0.6, kmax=4, ksqmax=16, seed=8))
+    v0 = np.random.default_rng(2).standard_normal((3, s.natom)) * np.sqrt(s.treq / s.masses())
+    dev = torch.device("cuda:0")
+    t = lambda a: torch.tensor(a, dtype=torch.float64, device=dev).contiguous()  # noqa: E731
+    eng = Engine.replicas([s], precision="fp64")
+    eng.set_list_skin(0.0)
+    start = [t(a) for a in (eng.packed_positions(), v0, eng.frclong()[0], eng.frcshort()[0])]
+    bufs = [b.clone() for b in start]
+    lt = torch.zeros(LONG_TERMS_BYTES // 8, dtype=torch.float64, device=dev)
+    st = torch.zeros(SHORT_TERMS_BYTES // 8, dtype=torch.float64, device=dev)
+    uk = torch.zeros(1, dtype=torch.float64, device=dev)
+
+    def reset():
+        if kind == "nvt":
+            eng.nvt_set(4.0 * s.natom, 2.0 * s.natom, s.treq, 3 * s.natom - 3)
+        for b, a in zip(bufs, start):
+            b.copy_(a)
+        for b in (lt, st, uk):
+            b.zero_()
+        torch.cuda.synchronize()
+
+    def run():
+        call = eng.nvt_run_device if kind == "nvt" else eng.vver_run_device
+        call(*bufs, 0.25 * s.delt, 2, 3, lt, st, uk, graph=False,
+             stream=torch.cuda.current_stream().cuda_stream)
+
+    print(f"case capture {kind}", flush=True)
+    reset()
+    run()
+    torch.cuda.synchronize()
+    want = [b.cpu() for b in (*bufs, lt, st, uk)]
+    g = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(g):
+        run()
+    kinds = _node_types(g)
+    assert set(kinds) <= {0, 5}, kinds     # kernels, and the empty nodes of joins
+    g.instantiate()
+    for _ in range(4):
+        reset()
+        g.replay()
+        torch.cuda.synchronize()
+        for b, w in zip((*bufs, lt, st, uk), want):
+            assert torch.equal(b.cpu().view(torch.int64), w.view(torch.int64))
+    eng.close()
