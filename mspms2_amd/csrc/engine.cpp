@@ -1503,7 +1503,7 @@ int enqueue_long(mspms_ctx* c, const double* x, const double* y, const double* z
         // rebuilt on the device)
         c->cb.half = (!grad && c->precision == MSPMS_PREC_MIXED) ? 1 : 0;
         launch_cluster_build(L, c->cb, x, y, z, fx, fy, fz, 0.25 * c->skin * c->skin,
-                             c->force_rebuild ? 1 : 0);
+                             c->force_rebuild ? 1 : 0, c->any_recip);
     }
     {
         ProfScope p(c, s, PROF_PAIR);

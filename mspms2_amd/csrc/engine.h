@@ -387,9 +387,11 @@ void launch_grid_node_major(hipStream_t s, const float* src, float* dst, size_t 
 // skin and reused while every atom stays within skin/2 of its position at
 // the build (force: rebuild regardless); reused calls only refresh the slot
 // positions.  A rebuild request made here is cleared by the finalize kernel.
+// beside: the Ewald kernels run on another stream meanwhile.
 void launch_cluster_build(const LaunchCtx& c, ClusterBufs& b, const double* x,
                           const double* y, const double* z, double* fx,
-                          double* fy, double* fz, double half_skin2, int force);
+                          double* fy, double* fz, double half_skin2, int force,
+                          bool beside);
 // gq/ge/gs: per-atom derivatives of the energy with respect to the atom's
 // own charge, epsilon and sigma (parameter adjoint, FP64); null: none
 void launch_pair(const LaunchCtx& c, const ClusterBufs& b, int precision,

@@ -788,7 +788,7 @@ __global__ void __launch_bounds__(256) k_plist(const int* __restrict__ ncl_total
 
 void launch_cluster_build(const LaunchCtx& c, ClusterBufs& b, const double* x, const double* y,
                           const double* z, double* fx, double* fy, double* fz, double half_skin2,
-                          int force) {
+                          int force, bool beside) {
     const int T = 256;
     int gA = (c.natom + T - 1) / T;
     const int nslot = b.maxcl * MSPMS_CL;
@@ -815,11 +815,14 @@ void launch_cluster_build(const LaunchCtx& c, ClusterBufs& b, const double* x, c
                            b.half, b.hist);
         // the last binning workgroup scans the cells.  1024 threads scan, and
         // arrive, faster where there are many (8,813 cells: 24.7 against 34.3 us;
-        // 6,144: 18.3 against 25.2); at 1,331 cells both take 13.0, and smaller
-        // systems would leave CUs idle while they bin.  But a workgroup of 16 waves
-        // also waits for a CU free of the side stream's work on the steps that
-        // build nothing (98,304 sites: 125 us behind the structure factors), so
-        // they are for calls that always build.
+        // 6,144: 18.3 against 25.2; a rebuild of 78,732 LJ sites 56 against 64,
+        // of 500,000 259 against 354, of 1,000,188 536 against 764, and the step that
+        // reuses its list the same); at 1,331 cells both take 13.0, and smaller
+        // systems would leave CUs idle while they bin.  But beside the Ewald
+        // kernels of the side stream a workgroup of 16 waves also waits for a free
+        // CU on the steps that build nothing (98,304 sites: 125 us behind the
+        // structure factors; 150,000: a step of 804 us grows by 2, a rebuild of
+        // 137 shrinks by 11), so there they are for calls that always build.
         auto bin = [&](auto kernel, int nt) {
             hipLaunchKernelGGL(kernel, dim3((c.natom + nt - 1) / nt), dim3(nt), 0, c.stream, c.natom,
                                x, y, z, c.atom_site, c.atom_mol, c.sites, c.mols, c.reps, b.atom_cell,
@@ -827,7 +830,7 @@ void launch_cluster_build(const LaunchCtx& c, ClusterBufs& b, const double* x, c
                                c.status, b.lstate, b.ncell, b.ncol, b.cell_start, b.col_cell0,
                                b.col_cl0, b.cl_col, b.ncl_total, b.maxcl, b.bin_ctr);
         };
-        if (b.ncell > 2048 && (force || half_skin2 == 0.0))
+        if (b.ncell > 2048 && (force || half_skin2 == 0.0 || !beside))
             bin(k_bin_scan<1024>, 1024);
         else
             bin(k_bin_scan<256>, 256);

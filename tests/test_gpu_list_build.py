@@ -66,3 +66,34 @@ def test_pairs_of_small_systems(name, precision):
             tol = 1e-12 if precision == "fp64" else 2e-5
             assert np.linalg.norm(f - fo) <= tol * np.linalg.norm(fo)
     eng.close()
+
+
+# with a skin, several passes of the cell scan: more than 8,192 cells by 1024
+# threads, and, beside the Ewald kernels, more than 4,096 by 256
+SKINNED = {
+    "lj-19652": lambda: configs.lj_fcc(ncell=17, jitter=0.05, seed=4),
+    "water-3375": lambda: configs.water_box(n_side=15, L=46.56, rc=8.0, kappa=0.35, kmax=3,
+                                            ksqmax=9, seed=4),
+}
+
+
+@pytest.mark.parametrize("name", list(SKINNED))
+def test_pairs_of_large_grids_with_a_skin(name):
+    s = system_of(SKINNED[name]())
+    print(f"{name} natom={s.natom}", flush=True)
+    eng = Engine(s, precision="fp64")
+    skin = (0.6 if name.startswith("water") else 0.2) / (
+        s.params["sigma_base"] if name.startswith("water") else 1.0)
+    eng.set_list_skin(skin)
+    eng.set_launch_shape(2.0, 4)
+    x = np.stack([s.xx, s.yy, s.zz])
+    u = np.random.default_rng(5).uniform(-1.0, 1.0, x.shape) / np.sqrt(3.0)
+    # a first build, a step that reuses the list, a rebuild
+    for d, builds in ((0.0, 1), (0.45 * skin, 1), (0.9 * skin, 2)):
+        g, t = eng.frclong(*(x + d * u))
+        assert eng.list_builds() == builds
+        f, to = Oracle(s).frclong(*(x + d * u))
+        for k in ("n_lj_pairs", "n_elec_pairs", "lj_pair_hash", "elec_pair_hash"):
+            assert t[k] == to[k], (d, k, t[k], to[k])
+        assert np.linalg.norm(g - f) <= 1e-12 * np.linalg.norm(f)
+    eng.close()
