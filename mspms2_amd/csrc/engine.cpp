@@ -119,6 +119,7 @@ struct mspms_ctx {
     bool any_intra = false, any_bonded = false, any_recip = false, any_sf = false;
     int max_mol_terms = 0;  // most bonded terms of one molecule (any species)
     int max_mol_intra = 0;  // most intramolecular pair terms
+    int max_rep_atoms = 0;  // the largest replica
     bool sf_split = false;  // the solid-fluid wall in frcshort / the inner loop
     bool any_vacuum = false, any_coul = false;
     int want_hash = -1;                  // -1: FP64 only
@@ -1252,9 +1253,12 @@ int build(mspms_ctx* c) {
     {
         // one partial of each kind per thread in the largest replica
         size_t most = 1;
-        for (const RepDev& R : c->reps)
+        c->max_rep_atoms = 0;
+        for (const RepDev& R : c->reps) {
             most = std::max({most, (size_t)R.natom, (size_t)R.nmol, (size_t)R.nk,
                              (size_t)(R.natom / MSPMS_CL + R.ncol + 1)});
+            c->max_rep_atoms = std::max(c->max_rep_atoms, R.natom);
+        }
         c->fin.nb = (int)std::min<size_t>(FIN_BLOCKS, (most + FIN_T - 1) / FIN_T);
     }
     HIPC(hipStreamSynchronize(s));
@@ -1520,8 +1524,14 @@ int enqueue_long(mspms_ctx* c, const double* x, const double* y, const double* z
                       (c->any_intra || recip_side);
     if (kicked) *kicked = fuse;
     // with the LJ pair forces alone there is nothing but the slot forces to add
-    // (80,000 sites: 10.6 us in two launches, 5.1 in the finalize pass)
-    const bool pair_only = !c->any_recip && !c->any_intra && !c->any_coul && !sf_long;
+    // (two replicas of 40,000 sites: 10.6 us in two launches, 5.1 in the finalize
+    // pass).  That pass has at most FIN_BLOCKS workgroups a replica: replicas
+    // of more than four sweeps of them fare better with a launch for all atoms
+    // (step of one replica, in the finalize pass and in launches of their own:
+    // 32,000 sites 50.7 and 52.1 us, 62,500 both 76, 78,732 91.9 and 90.3, 256,000
+    // 222 and 210, 1,000,188 913 and 827)
+    const bool pair_only = !c->any_recip && !c->any_intra && !c->any_coul && !sf_long &&
+                           c->max_rep_atoms <= 4 * FIN_BLOCKS * FIN_T;
     const bool defer = (recip_side || (pair_only && !grad)) && frec_deferred;
     if (frec_deferred) *frec_deferred = defer;
     if (defer) {
