@@ -100,6 +100,20 @@ def test_reciprocal_of_replicas_with_different_kmax():
         _check(s, fl, t)
 
 
+def test_reciprocal_of_many_small_replicas():
+    """180 replicas of up to five 64-atom tables, more than 512 tables in all:
+    chunks of several tables, most of them a whole replica."""
+    systems = [_system(20 + 7 * (r % 12), (3, 2, 3), 9, seed=r) for r in range(180)]
+    assert sum((s.natom + 63) // 64 for s in systems) > 512
+    print("case many replicas", flush=True)
+    eng = Engine.replicas(systems, precision="fp64")
+    f, terms = eng.frclong()
+    parts = eng.unpack(f)
+    eng.close()
+    for s, fl, t in zip(systems, parts, terms):
+        _check(s, fl, t)
+
+
 @pytest.mark.parametrize("nmol,kmax,ksq", [(40, (5, 6, 7), 49), (33, (6, 5, 11), 150),
                                            (22000, (1, 1, 9), 81)])
 def test_charge_derivative_matches_direct_sum(nmol, kmax, ksq):
