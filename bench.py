@@ -899,27 +899,28 @@ def main():
 
     g = mixed["groups"]
     natom = system.natom
-    nk = 2108
+    nk, nrow = 2108, 99
     # algorithmic work per launch (pair: 20 geometry + 24 LJ + 25 Ewald real
-    # FLOP-eq per i<j pair in range; reciprocal: 29 FP64 FLOP-eq per (k, atom)
-    # over the 1054 distinct +-k pairs: S(-k) = conj S(k) for real charges, so
-    # the other half of the reference's 2108 vectors is no work)
+    # FLOP-eq per i<j pair in range; reciprocal: 6 FP64 multiply-adds per
+    # (k, atom) of the two matrix products over the 1054 distinct +-k pairs,
+    # S(-k) = conj S(k) for real charges, so that the other half of the
+    # reference's 2108 vectors is no work; and 25 FLOP per ((kx, ky) row, atom))
     pair_flop = 20.0 * n_el + 24.0 * n_lj + 25.0 * n_el
-    recip_flop = 29.0 * (nk // 2) * natom
+    recip_flop = (12.0 * (nk // 2) + 25.0 * nrow) * natom
     wpc = mixed["tune"]["waves_per_cluster"]
     cand = {
-        "k_pair": (g.get("pair", 0.0), pair_flop, PEAK_FP32_TFLOPS,
+        "k_pair": (g.get("pair", 0.0), pair_flop, PEAK_FP32_TFLOPS, "valu",
                    ["k_pair_mx<1, %d, true, false>" % wpc]),
         "k_sk+k_sred+k_kforce": (g.get("recip_s", 0.0) + g.get("recip_f", 0.0), recip_flop,
-                                 PEAK_FP64_TFLOPS, ["k_sk<", "k_sred", "k_kforce<"]),
+                                 PEAK_FP64_TFLOPS, "matrix", ["k_sk<", "k_sred", "k_kforce<"]),
     }
     def roof(name):
-        kms, flop, peak, knames = cand[name]
+        kms, flop, peak, bound, knames = cand[name]
         achieved = flop / (kms * 1e-3) / 1e12 if kms > 0 else 0.0
         # HBM bytes per launch of the same kernels from the committed
         # counter summary (two rocprofv3 --pmc passes over `bench.py --probe`)
         traffic = traffic_of(knames)
-        return {"bound": "valu", "kernel": name, "achieved": achieved, "peak": peak,
+        return {"bound": bound, "kernel": name, "achieved": achieved, "peak": peak,
                 "unit": "TFLOP/s", "frac": achieved / peak, "traffic": traffic,
                 "traffic_unit": "bytes per launch", "flop_per_launch": flop,
                 "hbm_GBps_at_traffic": (traffic / (kms * 1e-3) / 1e9) if traffic else None,

@@ -14,10 +14,12 @@
 //   U = sum a_n c_n + b_n s_n, V, and U', V' with the weight n,
 // with E_r = C + i D, give D U + C V for the x and y components (times kx,
 // ky) and D U' + C V' for z: a (4 rows) x (2 kmaxz) by (2 kmaxz) x (atoms)
-// product and ten operations per (row, atom).  Both run on the FP64 matrix
-// instruction (v_mfma_f64_16x16x4): 12 multiply-adds per (k, atom) of the
-// half space and no recurrence along kz, where a lane per (row, kz segment)
-// and a lane per atom took 29 and were bound by their chains and by LDS and
+// product.  Both run on the FP64 matrix instruction (v_mfma_f64_16x16x4).  Per
+// row and n the first takes 4 multiply-adds an atom and the second 8, for the
+// two k's +n and -n: 6 multiply-adds, 12 FLOP, per (k, atom) of the half space,
+// and per (row, atom) 25 FLOP outside the products (E_r twice, the row's share
+// of the forces).  There is no recurrence along kz, where a lane per
+// (row, kz segment) and a lane per atom were bound by their chains and by LDS and
 // scalar loads per product.
 //
 //   k_sk     one workgroup per (replica, chunk of atoms): power tables of 64
