@@ -99,10 +99,15 @@ __device__ inline bool check_one(
     const float BIG = 3.0e38f;
     float lo[3] = {BIG, BIG, BIG}, hi[3] = {-BIG, -BIG, -BIG};
     if (live_cl) {
-        // (the charge in .w stays as the build left it)
-        double* px = reinterpret_cast<double*>(&slot_x64[t]);
-        *reinterpret_cast<double2*>(px) = make_double2(xo, yo);
-        px[2] = zo;
+        // the exact kernel's positions (the charge in .w stays as the build left
+        // it); the kernel of half lists reads the offsets alone, and a list of
+        // the other layout is built anew (960,000 LJ sites: 54.0 us with these
+        // stores, 45.4 without)
+        if (!half) {
+            double* px = reinterpret_cast<double*>(&slot_x64[t]);
+            *reinterpret_cast<double2*>(px) = make_double2(xo, yo);
+            px[2] = zo;
+        }
         const float4 off = make_float4((float)((w.x - C.x) + (xo - p0o.x)),
                                        (float)((w.y - C.y) + (yo - p0o.y)),
                                        (float)((w.z - C.z) + (zo - p0o.z)), (float)w.w);

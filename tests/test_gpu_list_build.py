@@ -97,3 +97,24 @@ def test_pairs_of_large_grids_with_a_skin(name):
             assert t[k] == to[k], (d, k, t[k], to[k])
         assert np.linalg.norm(g - f) <= 1e-12 * np.linalg.norm(f)
     eng.close()
+
+
+@pytest.mark.parametrize("nmol", [125, 512])     # built in one launch, and in five
+def test_half_and_full_lists_in_turn(nmol):
+    """The mixed kernel's half lists, whose reuse leaves the exact kernel's
+    positions as they were, and the adjoint's full lists on one engine: each
+    after moves of less than half the skin, forces against the oracle."""
+    s = system_of(configs.water_box(n_side=8, L=24.9, rc=8.0, kappa=0.35, kmax=3, ksqmax=9,
+                                    nmol=nmol, seed=4))
+    print(f"half and full lists {s.natom}", flush=True)
+    eng = Engine(s, precision="mixed")
+    skin = 1.0 / s.params["sigma_base"]
+    eng.set_list_skin(skin)
+    x = np.stack([s.xx, s.yy, s.zz])
+    u = np.random.default_rng(5).uniform(-1.0, 1.0, x.shape) / np.sqrt(3.0)
+    for k, exact in enumerate([False, False, True, True, False, False, True]):
+        xk = x + 0.07 * k * skin * u
+        g = eng.param_grad(*xk)[0] if exact else eng.frclong(*xk)[0]
+        f, _ = Oracle(s).frclong(*xk)
+        assert np.linalg.norm(g - f) <= (1e-12 if exact else 2e-5) * np.linalg.norm(f), (k, exact)
+    eng.close()
