@@ -80,7 +80,12 @@ extern "C" {
 #define MSPMS_EWALD_BC_VACUUM  2
 
 /* precision modes */
-#define MSPMS_PREC_FP64  0 /* reference operation order, FP64 everywhere      */
+#define MSPMS_PREC_FP64  0 /* FP64 everywhere: the reference's pair sets bit
+                              for bit and its operation order, but for sums
+                              over pairs and atoms, the Ewald and Wolf pair
+                              terms (own erfc) and, in device runs, the inner
+                              loops' bonds, angles and cosine dihedrals, all
+                              with no larger rounding error                   */
 #define MSPMS_PREC_MIXED 1 /* FP32 pair arithmetic, FP64 accumulation,
                               FP64 Ewald reciprocal and bonded terms          */
 

@@ -346,6 +346,9 @@ __global__ void __launch_bounds__(NT) k_bin_scan(
     // workgroup's writes, which the barrier orders before it: a fence by every
     // thread has each wave write back the XCD's L2 (70,508 atoms, 256
     // threads: 47.7 us with it, 34.3 without; 1024 threads: 43.9 and 24.7).
+    // What the last workgroup reads of the others are the counts alone, whose
+    // atomics every wave has waited for before the barrier: it needs the value
+    // they return (atom_slot).
     __shared__ int last;
     __shared__ int sh[32];
     __shared__ int stage[SCAN_LDS<NT>];

@@ -3,25 +3,27 @@
 // src/frclong.c:105-196 (ljfrc, ewald_real_frc, wolf_real_frc).
 //
 // A wave64 walks (part of) an i-cluster's row of the cluster-pair list.
-// Lane (i = lane>>3, j = lane&7) evaluates one site pair per j-cluster;
-// each i's force is reduced over its 8 lanes with wave shuffles at the end,
-// and the energy / virial partials over the whole wave.  For the exact
-// kernel the lists are full (both i->j and j->i), so every atom's force is
-// written once, without atomics, in a fixed order: the result is
-// deterministic.  The mixed kernel takes each cluster pair once and adds
+// Lane (i = lane>>3, j = lane&7) tests one site pair per j-cluster, and in
+// the mixed kernel evaluates it; in the exact one it evaluates the pairs that
+// the test queued for i.  Each i's force is reduced over its 8 lanes with wave
+// shuffles at the end, and the energy / virial partials over the whole wave.
+// For the exact kernel the lists are full (both i->j and j->i), so every
+// atom's force is written once, without atomics, in a fixed order: the result
+// is deterministic.  The mixed kernel takes each cluster pair once and adds
 // the j forces with FP64 atomics (half the pair terms; forces repeat to the
 // last bits).  Energies and virial reach the finalize doubled and are halved
 // there; pair counts and hashes are taken on i<j only.
-//   k_pair     exact mode: one wave per i-cluster
-//   k_pair_mx  mixed mode: WPC waves per i-cluster sharing its row, the
+//   k_pair     exact mode: WPC waves per i-cluster sharing its row, the
 //              partials combined through LDS in wave order
+//   k_pair_mx  mixed mode: likewise
 //
 // Precision modes:
 //   FP64   separation from the unwrapped FP64 positions with the reference's
-//          minimum image (d - L*rint(d/L), true division, no contraction),
-//          FP64 terms (LJ in the reference's order, Ewald and Wolf with the
-//          branch-free erfc of physics.h): the (i<j, r<rc) pair sets are
-//          those of src/frclong.c:114-125 bit for bit.
+//          minimum image (d - L*rint(d/L), the quotient by 1/L where that
+//          rounds to the same integer, no contraction), FP64 terms (LJ in the
+//          reference's order, Ewald and Wolf with the branch-free erfc of
+//          physics.h): the (i<j, r<rc) pair sets are those of
+//          src/frclong.c:114-125 bit for bit.
 //   MIXED  separation = (FP32 offset_i - offset_j) + (cluster-centre delta
 //          and image shift, FP64 rounded once to FP32); FP32 terms with the
 //          polynomial erfc; FP64 accumulation of forces, energies, virial.

@@ -2,7 +2,9 @@
 //
 // FP64 versions keep the reference's expression order with contraction
 // disabled, so that they round like the reference's x86-64 build; the libm
-// calls become ROCm device-library calls (erfc, exp: ~1 ulp).
+// calls become ROCm device-library calls (erfc, exp: ~1 ulp).  The exact pair
+// kernel takes Ewald and Wolf terms in another form (erfc_exp64, rsqrt_fma),
+// whose rounding error is smaller.
 // FP32 versions are the mixed-precision pair arithmetic.
 #pragma once
 #include <hip/hip_runtime.h>
