@@ -102,6 +102,8 @@ __attribute__((visibility("hidden"))) int mspms_fail(int code, const char* what)
 }
 
 // -------------------------------------------------------------------------
+constexpr int MAX_GRAPH_STEPS = 4;  // of a device run's graph (run_graph_steps)
+
 struct mspms_ctx {
     int device = 0, precision = MSPMS_PREC_MIXED;
     hipStream_t stream = nullptr;
@@ -256,14 +258,14 @@ struct mspms_ctx {
                    per == o.per;
         }
     };
-    // device runs captured as graphs, one step (or move) and RUN_GRAPH_STEPS
-    // steps, each valid for its kind and arguments until the next build
+    // device runs captured as graphs of 1 to MAX_GRAPH_STEPS steps (or one
+    // move), each valid for its kind and arguments until the next build
     struct Graph {
         hipGraph_t graph = nullptr;
         hipGraphExec_t exec = nullptr;
         int kind = -1;  // GRAPH_*
         GraphKey key{};
-    } graphs[2];
+    } graphs[MAX_GRAPH_STEPS];
 };
 
 namespace {
@@ -285,7 +287,7 @@ enum { GRAPH_VVER = 0, GRAPH_HMC = 1, GRAPH_NVT = 2, GRAPH_NPT = 3 };
 template <typename F>
 int ensure_graph(mspms_ctx* c, hipStream_t s, int kind, const mspms_ctx::GraphKey& key,
                  F&& enqueue) {
-    mspms_ctx::Graph& G = c->graphs[key.per > 1];
+    mspms_ctx::Graph& G = c->graphs[key.per - 1];
     if (G.exec && key == G.key && G.kind == kind) return 0;
     drop_graph(G);
     // the capture stream must not have work in flight from the caller
@@ -1633,34 +1635,32 @@ int enqueue_vver(mspms_ctx* c, double* pos, double* vel, double* fl, double* fs,
     return 0;
 }
 
-// Steps of the longer of a device run's two graphs.  Four steps in one graph
-// drop three of the four graph boundaries per four steps (0.6 us per step at
-// the 12,288-site water step of ~97 us); the steps that four does not divide
-// replay a graph of one step (enqueued kernel by kernel they take about 16 us
-// more each: 6 NVT steps of 12,288 sites 943 us, 910 as six graphs).  Both
-// graphs stay, whatever length the next run has: a program that runs 10, 9
-// and 8 steps in turn captures each once.
-constexpr int RUN_GRAPH_STEPS = 4;
-
-// How many steps of a run go by graphs of RUN_GRAPH_STEPS: short runs that need
-// the graph of one step anyway take that alone, since capturing the longer
-// one as well costs a first run of 10 steps about 70 us (3,009 sites) and
-// saves each later one about 4.
-int long_graph_steps(int nsteps) {
-    if (nsteps < 4 * RUN_GRAPH_STEPS && nsteps % RUN_GRAPH_STEPS) return 0;
-    return nsteps - nsteps % RUN_GRAPH_STEPS;
+// Steps per graph of a device run: four in one graph drop three of the four
+// graph boundaries per four steps (0.6 us per step at the 12,288-site water
+// step of ~97 us).  What the count leaves over replays a graph of one step
+// (enqueued kernel by kernel such steps take about 16 us more each: 6 NVT steps
+// of 12,288 sites 943 us, 910 as six graphs).  Runs of fewer than 16 steps take
+// the largest count that leaves none over, since capturing a second graph
+// costs a first run of 10 steps about 150 us and saves each later one few (3,009
+// sites: 1084 us by graphs of four and one, 1086 of two, 1094 of one).
+// The graphs of each count stay, whatever length the next run has: a program
+// that runs 10, 9 and 8 steps in turn captures each once.
+int run_graph_steps(int nsteps) {
+    if (nsteps >= 4 * MAX_GRAPH_STEPS) return MAX_GRAPH_STEPS;
+    int per = MAX_GRAPH_STEPS;
+    while (per > 1 && (nsteps < per || nsteps % per)) per--;
+    return per;
 }
 
-// the graphs that nsteps steps need
+// the graphs of `per` steps and, for what that leaves over, of one
 template <typename F>
 int ensure_run_graphs(mspms_ctx* c, hipStream_t s, int kind, mspms_ctx::GraphKey key, int nsteps,
-                      F&& enqueue) {
-    const int by_long = long_graph_steps(nsteps);
-    int rc = 0;
-    for (int per : {RUN_GRAPH_STEPS, 1}) {
-        key.per = per;
-        if (!rc && (per > 1 ? by_long > 0 : by_long < nsteps))
-            rc = ensure_graph(c, s, kind, key, enqueue);
+                      int per, F&& enqueue) {
+    key.per = per;
+    int rc = nsteps >= per ? ensure_graph(c, s, kind, key, enqueue) : 0;
+    if (!rc && nsteps % per != 0) {
+        key.per = 1;
+        rc = ensure_graph(c, s, kind, key, enqueue);
     }
     return rc;
 }
@@ -1933,8 +1933,8 @@ extern "C" int mspms_vver_step_device(mspms_ctx* c, double* pos, double* vel, do
     return enqueue_vver(c, pos, vel, fl, fs, delt, nstep_inner, lterms, sterms, ukin, s);
 }
 
-// nsteps RESPA outer steps; with use_graph graphs of RUN_GRAPH_STEPS steps and
-// of one step, captured once (on the context stream), are replayed on
+// nsteps RESPA outer steps; with use_graph graphs of a few steps and of one step
+// (run_graph_steps), captured once (on the context stream), are replayed on
 // `stream`.  Optional histories receive each step's terms (nsteps * nrep
 // entries) and kinetic energies (nsteps * nrep doubles).
 extern "C" int mspms_vver_run_device(mspms_ctx* c, double* pos, double* vel, double* fl,
@@ -1950,9 +1950,10 @@ extern "C" int mspms_vver_run_device(mspms_ctx* c, double* pos, double* vel, dou
     HIPC(hipSetDevice(c->device));
     hipStream_t s = stream ? (hipStream_t)stream : c->stream;
     const int nr = c->nrep;
+    const int per = run_graph_steps(nsteps);
     if (use_graph) {
         mspms_ctx::GraphKey k{pos, vel, fl, fs, lterms, sterms, ukin, delt, nstep_inner};
-        int rc = ensure_run_graphs(c, s, GRAPH_VVER, k, nsteps, [&](hipStream_t cs) {
+        int rc = ensure_run_graphs(c, s, GRAPH_VVER, k, nsteps, per, [&](hipStream_t cs) {
             return enqueue_vver(c, pos, vel, fl, fs, delt, nstep_inner, lterms, sterms, ukin, cs);
         });
         if (rc) return rc;
@@ -1993,8 +1994,8 @@ extern "C" int mspms_vver_run_device(mspms_ctx* c, double* pos, double* vel, dou
         hist_off.on = true;
     }
     for (int t = 0; t < nsteps;) {
-        const bool grp = use_graph && t < long_graph_steps(nsteps);
-        const int adv = grp ? RUN_GRAPH_STEPS : 1;
+        // graphs of `per` steps while that many remain, then single steps
+        const int adv = use_graph && nsteps - t >= per ? per : 1;
         if (gate && t + adv >= nsteps) {
             // the launch that holds the last step reduces its terms (the
             // other steps of a graph reduce theirs too: the last one wins)
@@ -2002,7 +2003,7 @@ extern "C" int mspms_vver_run_device(mspms_ctx* c, double* pos, double* vel, dou
         }
         t += adv;
         if (use_graph) {
-            HIPC(hipGraphLaunch(c->graphs[grp].exec, s));
+            HIPC(hipGraphLaunch(c->graphs[adv - 1].exec, s));
         } else {
             int rc = enqueue_vver(c, pos, vel, fl, fs, delt, nstep_inner, lterms, sterms, ukin, s);
             if (rc) return rc;
@@ -2411,9 +2412,10 @@ extern "C" int mspms_nvt_run_device(mspms_ctx* c, double* pos, double* vel, doub
     hipStream_t s = stream ? (hipStream_t)stream : c->stream;
     // graphs of several steps, and the terms of the last step only, as in
     // the NVE run
+    const int per = run_graph_steps(nsteps);
     if (use_graph) {
         mspms_ctx::GraphKey k{pos, vel, fl, fs, lterms, sterms, ukin, delt, nstep_inner};
-        int rc = ensure_run_graphs(c, s, GRAPH_NVT, k, nsteps, [&](hipStream_t cs) {
+        int rc = ensure_run_graphs(c, s, GRAPH_NVT, k, nsteps, per, [&](hipStream_t cs) {
             return enqueue_nvt(c, pos, vel, fl, fs, delt, nstep_inner, lterms, sterms, ukin, cs);
         });
         if (rc) return rc;
@@ -2422,11 +2424,11 @@ extern "C" int mspms_nvt_run_device(mspms_ctx* c, double* pos, double* vel, doub
     FinGate fin{c, s};
     if (nsteps > 1) HIPC(fin.set(false));
     for (int t = 0; t < nsteps;) {
-        const bool grp = use_graph && t < long_graph_steps(nsteps);
-        t += grp ? RUN_GRAPH_STEPS : 1;
+        const int adv = use_graph && nsteps - t >= per ? per : 1;
+        t += adv;
         if (fin.closed && t >= nsteps) HIPC(fin.set(true));
         if (use_graph) {
-            HIPC(hipGraphLaunch(c->graphs[grp].exec, s));
+            HIPC(hipGraphLaunch(c->graphs[adv - 1].exec, s));
         } else {
             int rc = enqueue_nvt(c, pos, vel, fl, fs, delt, nstep_inner, lterms, sterms, ukin, s);
             if (rc) return rc;

@@ -1,5 +1,5 @@
-"""NVE and NVT device runs whose step counts give graphs of one and four steps,
-both, and terms reduced for the last step only: the same state and
+"""NVE and NVT device runs whose step counts give graphs of one to four steps,
+and of two counts, and terms reduced for the last step only: the same state and
 the same terms as one-step calls without graphs.  FP64, whose sums all have a
 fixed order, so the two differ by nothing."""
 import numpy as np
