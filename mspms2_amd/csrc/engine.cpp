@@ -1951,6 +1951,10 @@ extern "C" int mspms_vver_run_device(mspms_ctx* c, double* pos, double* vel, dou
     hipStream_t s = stream ? (hipStream_t)stream : c->stream;
     const int nr = c->nrep;
     const int per = run_graph_steps(nsteps);
+    // the run's own buffers take the snapshot back after an overflow, also where
+    // its steps replay graphs captured earlier
+    c->snap_pos = pos;
+    c->snap_vel = vel;
     if (use_graph) {
         mspms_ctx::GraphKey k{pos, vel, fl, fs, lterms, sterms, ukin, delt, nstep_inner};
         int rc = ensure_run_graphs(c, s, GRAPH_VVER, k, nsteps, per, [&](hipStream_t cs) {
@@ -2182,6 +2186,8 @@ extern "C" int mspms_hmc_run_device(mspms_ctx* c, double* pos, double* vel, doub
         return fail(MSPMS_EINVAL, "null argument");
     HIPC(hipSetDevice(c->device));
     hipStream_t s = stream ? (hipStream_t)stream : c->stream;
+    c->snap_pos = pos;  // as in the NVE run
+    c->snap_vel = vel;
     if (use_graph) {
         mspms_ctx::GraphKey k{pos, vel, fl, fs, lterms, sterms, ukin, delt,
                               nstep_inner * 65536 + nmd};

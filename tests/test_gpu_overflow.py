@@ -71,3 +71,41 @@ def test_overflow_restores_run_start_and_repeat_matches(graph):
     assert np.abs(x - want_x).max() <= 1e-12 * np.abs(want_x).max()
     assert np.abs(v - want_v).max() <= 1e-12 * np.abs(want_v).max()
     eng.close()
+
+
+@pytest.mark.parametrize("graph", [True, False])
+def test_overflow_of_a_replayed_run_restores_its_own_buffers(graph):
+    """Two runs of one engine on buffers of their own, of different lengths, so
+    that each has its captured graph; the first again, without a new capture,
+    from positions too dense for the lists: its buffers are put back, and the
+    other run's stay as they are."""
+    import torch
+    dev = torch.device("cuda:0")
+    s = system_of(configs.lj_fcc(ncell=6, rho=0.25, rc=2.5, jitter=0.02, seed=3))
+    x = np.stack([s.xx, s.yy, s.zz])
+    dense = x * (0.25 / 0.8442) ** (1.0 / 3.0)
+    eng = Engine(s, precision="fp64")
+    # rows that hold the dilute fluid's pairs (32 entries) but not the dense one's (64)
+    eng.set_list_capacity(48)
+    a, b = _buffers(eng, s, dev), _buffers(eng, s, dev)
+
+    def run(bufs, n):
+        pos, vel, fl, fs, lt, st, uk = bufs
+        torch.cuda.synchronize()
+        eng.vver_run_device(pos, vel, fl, fs, s.delt, 1, n, lt, st, uk, graph=graph)
+
+    print(f"case replayed run graph={graph}", flush=True)
+    run(a, 4)
+    eng.sync()
+    run(b, 1)
+    eng.sync()
+    xb, vb = b[0].cpu().numpy(), b[1].cpu().numpy()
+    a[0].copy_(torch.tensor(dense, device=dev))
+    va = a[1].cpu().numpy()
+    run(a, 4)
+    with pytest.raises(EngineError) as e:
+        eng.sync()
+    assert "ENOMEM" in str(e.value) and "restored" in str(e.value) and "step 1" in str(e.value)
+    assert np.array_equal(a[0].cpu().numpy(), dense) and np.array_equal(a[1].cpu().numpy(), va)
+    assert np.array_equal(b[0].cpu().numpy(), xb) and np.array_equal(b[1].cpu().numpy(), vb)
+    eng.close()
