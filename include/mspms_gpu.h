@@ -411,9 +411,11 @@ int mspms_vver_step_device(mspms_ctx* ctx, double* pos, double* vel, double* fl,
                            double* ukin, void* stream);
 
 /* nsteps calls of mspms_vver_step_device with the same arguments.  With
- * use_graph != 0 one outer step (all kernels of every replica) is captured
- * once as a HIP graph on the context stream and replayed on `stream`; the
- * graph is kept for the same argument set until the system is rebuilt.
+ * use_graph != 0 one to four outer steps (all kernels of every replica) are
+ * captured as a HIP graph on the context stream and replayed on `stream`; the
+ * latest graph of each count is kept for its arguments until the system is
+ * rebuilt.  Without it the call enqueues kernels only (and, for histories,
+ * may allocate), so that a caller can capture it.
  * lhist / shist / ukin_hist (device, optional) receive every step's terms
  * and kinetic energies, nsteps * nreplica entries, step-major: each step's
  * closing reduction pass appends them itself (no copy per step), which is
@@ -478,8 +480,8 @@ int mspms_hmc_draw(mspms_ctx* ctx, int replica, int n, double* out);
  * nsteps steps of every replica from pos / vel with fl / fs holding the
  * long and short forces of pos (as after the reference's start-up
  * frclong / frcshort), leaving lterms / sterms of the last step and ukin
- * [nrep]; replayed from one captured graph when use_graph is set.
- * mspms_nvt_get downloads the states (thermostat variables, energies
+ * [nrep]; replayed from captured graphs when use_graph is set, as
+ * mspms_vver_run_device.  mspms_nvt_get downloads the states (thermostat variables, energies
  * unhts / unhtss, ukin, tinst = 2 ukin / nfree). */
 typedef struct mspms_nvt_state {
     double qq, qqs;            /* thermostat masses (outer, inner)          */

@@ -297,7 +297,7 @@ class Engine:
 
     def vver_run_device(self, pos, vel, fl, fs, delt, nstep_inner, nsteps, lterms, sterms, ukin,
                         lhist=None, shist=None, ukin_hist=None, graph=True, stream=None):
-        """nsteps RESPA outer steps; graph=True replays one captured step."""
+        """nsteps RESPA outer steps; graph=True replays captured steps."""
         p = self._ptr
         _check(lib().mspms_vver_run_device(
             self._h, p(pos), p(vel), p(fl), p(fs), float(delt), int(nstep_inner), int(nsteps),
