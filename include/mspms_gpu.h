@@ -481,8 +481,8 @@ int mspms_hmc_draw(mspms_ctx* ctx, int replica, int n, double* out);
  * long and short forces of pos (as after the reference's start-up
  * frclong / frcshort), leaving lterms / sterms of the last step and ukin
  * [nrep]; replayed from captured graphs when use_graph is set, as
- * mspms_vver_run_device.  mspms_nvt_get downloads the states (thermostat variables, energies
- * unhts / unhtss, ukin, tinst = 2 ukin / nfree). */
+ * mspms_vver_run_device.  mspms_nvt_get downloads the states (thermostat
+ * variables, energies unhts / unhtss, ukin, tinst = 2 ukin / nfree). */
 typedef struct mspms_nvt_state {
     double qq, qqs;            /* thermostat masses (outer, inner)          */
     double gg, ggs;            /* thermostat degrees of freedom (nfree)     */
