@@ -222,7 +222,6 @@ struct mspms_ctx {
     std::vector<long> prof_n;          // recorded launches per group
     bool capturing = false;            // no event records inside a capture
 
-
     // batched HMC chains (mspms_hmc_init)
     DevBuf<RanmarDev> d_rng;
     DevBuf<HmcRep> d_hmc;
@@ -289,10 +288,11 @@ int ensure_graph(mspms_ctx* c, hipStream_t s, int kind, const mspms_ctx::GraphKe
                  F&& enqueue) {
     mspms_ctx::Graph& G = c->graphs[key.per - 1];
     if (G.exec && key == G.key && G.kind == kind) return 0;
-    drop_graph(G);
-    // the capture stream must not have work in flight from the caller
+    // the capture stream must not have work in flight from the caller, and the
+    // graph that is replaced must have run
     HIPC(hipStreamSynchronize(s));
     HIPC(hipStreamSynchronize(c->stream));
+    drop_graph(G);
     c->capturing = true;
     HIPC(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
     int rc = 0;
